@@ -141,7 +141,7 @@ int rgpu_bvh_export(const rgpu_bvh* bvh, float* bounds, int32_t* left, int32_t* 
 
 /* ---------------------------------------------------------------- scene (device)
  * Replaces SceneManager::createBuffer (common/scene_manager.hpp:579-591) and the
- * SceneBuffer it fills (common/scene_manager.hpp:284-294): packs the stackless node
+ * SceneBuffer it fills (common/scene_manager.hpp:284-294): packs the stackless walk
  * records, the threaded node tables (one per ray-direction class and one for the single-table
  * walk, each in its own pre-order) and the primitive records, and uploads them with the
  * vertices. Host arrays are copied; the caller keeps ownership. A BVH of 2^30 nodes or more
@@ -168,13 +168,14 @@ int rgpu_extension_ray_cast(rgpu_ctx* ctx, rgpu_stream stream, const rgpu_scene*
 /* Launch shape of the persistent ray-cast kernel used when block == 0: resident waves per
  * SIMD (grid = CUs * waves_per_simd workgroups of 256; 1..16), the number of idle lanes of a
  * wave that makes it hand out its next rays (1..64), and the number of lanes waiting at leaves
- * that makes it test their primitives (1..64). 0 keeps the default (8 waves; refill at 24 idle
- * lanes for stackless, 48 for threaded; leaves at 8 waiting lanes for stackless, 6 for threaded,
- * or once as many lanes wait as walk on). leaf_batch also applies to the one-thread-per-ray kernels (block != 0), whose
+ * that makes it test their primitives (1..64). 0 keeps the default (7 waves for stackless, 8 for
+ * threaded; refill at 24 idle lanes for stackless, 48 for threaded; leaves at 12 waiting lanes for
+ * stackless, 6 for threaded, or once as many lanes wait as walk on). leaf_batch also applies to
+ * the one-thread-per-ray kernels (block != 0), whose
  * default is 64 (leaves only once as many lanes wait as walk on) and where 1 selects the plain
- * one-ray walk. treelet: the number of top-of-tree stackless node records each
- * workgroup of the persistent kernel copies to LDS and reads from there (1..1024, 64 bytes
- * each; 0 = default 320; RGPU_TREELET_OFF = none). Results do not depend on any of them. No
+ * one-ray walk. treelet: the number of top-of-tree stackless walk records each
+ * workgroup of the persistent kernel copies to LDS and reads from there (1..1024, 112 bytes
+ * each, as many as fit; 0 = default 128; RGPU_TREELET_OFF = none). Results do not depend on any of them. No
  * counterpart in the reference (it leaves launch shapes to the OpenCL driver,
  * common/raccoon_ocl.hpp:906). */
 #define RGPU_TREELET_OFF 0xFFFFFFFFu

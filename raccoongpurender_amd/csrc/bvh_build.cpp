@@ -372,6 +372,65 @@ void mark_leaf_links(std::vector<SLNode>* nodes) {
     }
 }
 
+uint32_t pack_walk(const BVHTree& t, uint32_t top, std::vector<WalkNode>* out) {
+    const std::vector<BuildNode>& nodes = t.nodes;
+    const size_t nn = nodes.size();
+    out->clear();
+    if (nn == 0) return kInvalid;
+    auto branch = [&](int32_t i) { return nodes[i].left >= 0; };
+    auto word = [&](int32_t i) {
+        return kLeafFlag | ((nodes[i].prim_cnt - 1) << 28) | nodes[i].prim_beg;
+    };
+    if (!branch(0)) return word(0);
+    // the grandchildren of a record's node, the children of a leaf child being itself
+    auto family = [&](int32_t i, int32_t g[4]) {
+        const int32_t kids[2] = {nodes[i].left, nodes[i].right};
+        for (int k = 0; k < 2; ++k) {
+            g[2 * k] = branch(kids[k]) ? nodes[kids[k]].left : kids[k];
+            g[2 * k + 1] = branch(kids[k]) ? nodes[kids[k]].right : kids[k];
+        }
+    };
+    // parents precede their children in the tree's order: depth parity, then the ids
+    std::vector<uint8_t> odd(nn, 0);
+    std::vector<uint32_t> id(nn, kInvalid);
+    std::vector<int32_t> order;  // record id -> node
+    for (size_t i = 0; i < nn; ++i)
+        if (branch((int32_t)i)) odd[nodes[i].left] = odd[nodes[i].right] = odd[i] ^ 1;
+    order.push_back(0);
+    id[0] = 0;
+    for (size_t h = 0; h < order.size() && order.size() < top; ++h) {
+        int32_t g[4];
+        family(order[h], g);
+        for (int k = 0; k < 4 && order.size() < top; ++k)
+            if (branch(g[k]) && !odd[g[k]] && id[g[k]] == kInvalid) {
+                id[g[k]] = (uint32_t)order.size();
+                order.push_back(g[k]);
+            }
+    }
+    for (size_t i = 0; i < nn; ++i)
+        if (!odd[i] && id[i] == kInvalid && branch((int32_t)i)) {
+            id[i] = (uint32_t)order.size();
+            order.push_back((int32_t)i);
+        }
+    out->resize(order.size());
+    for (size_t r = 0; r < order.size(); ++r) {
+        WalkNode& w = (*out)[r];
+        int32_t g[4];
+        family(order[r], g);
+        for (int k = 0; k < 4; ++k) {
+            for (int a = 0; a < 3; ++a) {
+                w.box[k][a] = nodes[g[k]].bmin[a];
+                w.box[k][3 + a] = nodes[g[k]].bmax[a];
+            }
+            w.link[k] = branch(g[k]) ? 8 * id[g[k]] : word(g[k]);
+            w.pad[k] = 0;
+        }
+        for (int k = 0; k < 4; k += 2)
+            if (g[k] == g[k + 1]) w.link[k + 1] = kInvalid;  // a leaf child
+    }
+    return 0;
+}
+
 void pack_threaded(const BVHTree& t, std::vector<MTNode>* out) {
     const uint32_t nn = (uint32_t)t.nodes.size();
     out->assign((size_t)kMTOrders * nn, MTNode());

@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstring>
 #include <exception>
+#include <future>
 #include <mutex>
 #include <new>
 #include <stdexcept>
@@ -355,18 +356,24 @@ int rgpu_scene_create(rgpu_ctx* ctx, const rgpu_bvh* bvh, const float* points, u
     std::vector<SLNode> sl;
     std::vector<MTNode> mt;
     std::vector<PrimRec> pr;
+    std::vector<WalkNode> walk;
+    // beside the other packers (its future waits for it on every way out)
+    std::future<uint32_t> packed =
+        std::async(std::launch::async, [&] { return pack_walk(bvh->tree, kTreeletMaxNodes, &walk); });
     pack_stackless(bvh->tree, &sl);
     number_top_breadth_first(&sl, kTreeletMaxNodes);
     mark_leaf_links(&sl);
+    const uint64_t sl_print = fingerprint64(sl.data(), sl.size() * sizeof(SLNode), ntris);
     pack_threaded(bvh->tree, &mt);
     pack_prims(bvh->tree, points, stride, indices, ntris, spheres, nspheres, &pr);
     std::vector<float> p4((size_t)npoints * 4, 0.0f);
     for (uint32_t i = 0; i < npoints; ++i)
         for (int k = 0; k < 3; ++k) p4[4 * (size_t)i + k] = points[(size_t)i * stride + k];
+    const uint32_t root = packed.get();
     rgpu_scene* s = new rgpu_scene();
     s->ctx = ctx;
     int rc = RGPU_OK;
-    if (rc == RGPU_OK) rc = upload_new(ctx, sl.data(), sl.size() * sizeof(SLNode), &s->sl);
+    if (rc == RGPU_OK) rc = upload_new(ctx, walk.data(), walk.size() * sizeof(WalkNode), &s->sl);
     if (rc == RGPU_OK) rc = upload_new(ctx, mt.data(), mt.size() * sizeof(MTNode), &s->mt);
     if (rc == RGPU_OK) rc = upload_new(ctx, pr.data(), pr.size() * sizeof(PrimRec), &s->prims);
     if (rc == RGPU_OK) rc = upload_new(ctx, p4.data(), p4.size() * sizeof(float), &s->points);
@@ -376,27 +383,29 @@ int rgpu_scene_create(rgpu_ctx* ctx, const rgpu_bvh* bvh, const float* points, u
         rgpu_scene_destroy(s);
         return rc;
     }
-    s->dev.sl_nodes = (const SLNode*)s->sl;
+    s->dev.walk_nodes = (const WalkNode*)s->sl;
+    s->dev.nwalk = (uint32_t)walk.size();
     s->dev.mt_nodes = (const MTNode*)s->mt;
     s->dev.prims = (const PrimRec*)s->prims;
     s->dev.points = (const float4*)s->points;
     s->dev.indices = (const uint32_t*)s->indices;
     s->dev.spheres = (const float4*)s->spheres;
+    s->dev.root = root;
     s->dev.nnodes = (uint32_t)bvh->tree.nodes.size();
     s->dev.sphere_begin = (int32_t)ntris;
     bool finite = true;
     for (const BuildNode& b : bvh->tree.nodes)
-        for (int k = 0; k < 3; ++k) finite = finite && std::isfinite(b.bmin[k]) && std::isfinite(b.bmax[k]);
+        for (int k = 0; k < 3; ++k)
+            finite = finite && std::isfinite(b.bmin[k]) && std::isfinite(b.bmax[k]) && b.bmin[k] <= b.bmax[k];
     s->dev.boxes_finite = finite ? 1u : 0u;
     s->nprims = ntris + nspheres;
-    s->fingerprint = fingerprint64(pr.data(), pr.size() * sizeof(PrimRec),
-                                   fingerprint64(sl.data(), sl.size() * sizeof(SLNode), ntris));
+    s->fingerprint = fingerprint64(pr.data(), pr.size() * sizeof(PrimRec), sl_print);
     if (!bvh->tree.nodes.empty())
         for (int k = 0; k < 3; ++k) {
             s->lo[k] = bvh->tree.nodes[0].bmin[k];
             s->hi[k] = bvh->tree.nodes[0].bmax[k];
         }
-    s->bytes[0] = sl.size() * sizeof(SLNode);
+    s->bytes[0] = walk.size() * sizeof(WalkNode);
     s->bytes[1] = mt.size() * sizeof(MTNode);
     s->bytes[2] = pr.size() * sizeof(PrimRec);
     s->bytes[3] = p4.size() * sizeof(float) + (size_t)ntris * 12 + (size_t)nspheres * 16;

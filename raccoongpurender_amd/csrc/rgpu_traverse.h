@@ -28,7 +28,9 @@ enum { kVariantStackless = 0, kVariantThreaded = 1, kVariantSingleThreaded = 2 }
 
 // Device-resident scene as the kernels see it.
 struct TraceScene {
-    const SLNode* sl_nodes = nullptr;
+    const WalkNode* walk_nodes = nullptr;  // the stackless walk's records
+    uint32_t nwalk = 0;
+    uint32_t root = 0;  // the root's walk link: its record, or the word of a root leaf
     const MTNode* mt_nodes = nullptr;  // kMTOrders tables of nnodes records
     const PrimRec* prims = nullptr;
     const float4* points = nullptr;    // original vertices (for geometric normals)
@@ -36,15 +38,14 @@ struct TraceScene {
     const float4* spheres = nullptr;
     uint32_t nnodes = 0;
     int32_t sphere_begin = 0;
-    uint32_t boxes_finite = 0;  // every node box finite (the slab test may drop its NaN guard)
+    uint32_t boxes_finite = 0;  // every node box finite and ordered (the slab test may drop its NaN guard)
 };
 
 // Launch shape of the persistent ray-cast kernel: CUs to fill, resident waves per SIMD (grid =
 // cu_count * waves_per_simd workgroups of 256), the idle-lane count that triggers a refill and
 // the count of lanes waiting at leaves that triggers their primitive tests. Zeros take the
-// defaults (256 CUs, 8 waves; refill at 24 lanes for the stackless walk, 48 for the threaded
-// ones; leaves at 8 waiting lanes for the stackless walk, 6 for the threaded ones), measured on
-// 4M incoherent rays over 1.3M triangles.
+// defaults (256 CUs; 7 waves, refill at 24 lanes and leaves at 12 waiting lanes for the stackless
+// walk, 8, 48 and 6 for the threaded ones), measured on 4M incoherent rays over 1.3M triangles.
 struct TraceTuning {
     uint32_t cu_count = 0;
     uint32_t waves_per_simd = 0;
@@ -53,15 +54,27 @@ struct TraceTuning {
     uint32_t treelet = 0;  // stackless records staged in LDS per workgroup; kTreeletOff: none
 };
 constexpr uint32_t kDefaultLeafBatch = 6;
-constexpr uint32_t kDefaultLeafBatchStackless = 8;
+constexpr uint32_t kDefaultLeafBatchStackless = 12;
+constexpr uint32_t kDefaultWavesStackless = 7;
 // One thread per ray (coherent rays, the wavefront's per-slot trace): leaves wait until as many
 // lanes wait as walk on.
 constexpr uint32_t kPerRayLeafBatch = 64;
 // The scene packer numbers this many top records breadth-first, so that any LDS treelet of up
-// to this size is a prefix of the node array (64 KB of LDS).
+// to this size is a prefix of the record array.
 constexpr uint32_t kTreeletMaxNodes = 1024;
 constexpr uint32_t kTreeletOff = 0xFFFFFFFFu;
-constexpr uint32_t kDefaultTreelet = 320;
+constexpr uint32_t kDefaultTreelet = 128;
+// Stack entries of a stackless walk in LDS, one column per lane, and behind them in private
+// memory: a walk defers at most one link per level, and leaves lie at depth 64 at most.
+constexpr uint32_t kWalkStackLds = 8;
+constexpr uint32_t kWalkStackSpill = 64 - kWalkStackLds;
+constexpr uint32_t kStagedBytes = 112;  // of a walk record in LDS
+// Dynamic LDS of a kernel that walks stackless records: staged records, then the stacks.
+constexpr size_t walk_lds_bytes(uint32_t top, uint32_t threads) {
+    return (size_t)top * kStagedBytes + (size_t)threads * kWalkStackLds * 4u;
+}
+// (a launch of 256 threads stages at most what 64 KB leave beside the stacks)
+constexpr uint32_t kTreeletMaxStaged = (65536u - 256u * kWalkStackLds * 4u) / kStagedBytes;
 
 // counters: null for the production kernels; otherwise 5 device u64 totals
 // {branch visits, leaf visits, parent steps, primitive tests, threaded node visits}.

@@ -7,7 +7,8 @@
 
 namespace rgpu {
 
-// Stackless (parent-pointer) BVH2 record, one per node, indexed by the node's
+// Stackless (parent-pointer) BVH2 record of the host packer (fingerprints of a scene are taken
+// over it; the device walks WalkNode records), one per node, indexed by the node's
 // depth-first pre-order id (the numbering of common/stackless_bvh.hpp:283-292).
 // Replaces the reference's 96-byte StacklessBVHNode (common/stackless_bvh.hpp:264-275,
 // kernels/extension_ray_cast_stackless.cl:21-32): the child boxes are stored as
@@ -39,6 +40,24 @@ static_assert(sizeof(SLNode) == 64, "stackless node record must be 64 bytes");
 static const uint32_t kLeafFlag = 0x80000000u;
 static const uint32_t kChildLeaf = 0x40000000u;
 static const uint32_t kInvalid = 0xFFFFFFFFu;
+
+// Record of the stackless walk on the device, one 128-byte line per branch node at an even depth:
+// the boxes of its four grandchildren (6 floats each, min xyz then max xyz; left child's first)
+// and their links. A link is
+//   a branch's   8 * its record's id (the record's index in 16-byte units); kFirstHalf or
+//                kSecondHalf added means that child of the record's node alone;
+//   a leaf's     kLeafFlag | ((count - 1) << 28) | first slot, its primitive word (never all ones:
+//                first + count <= 2^28 - 1).
+// A child that is a leaf itself fills both of its boxes with its own and has kInvalid for its
+// second link. Record ids stay below 2^28 (a tree has fewer than 2^28 primitives).
+struct alignas(128) WalkNode {
+    float box[4][6];
+    uint32_t link[4];
+    uint32_t pad[4];
+};
+static_assert(sizeof(WalkNode) == 128, "walk record must be one 128-byte line");
+static const uint32_t kFirstHalf = 1;
+static const uint32_t kSecondHalf = 2;
 
 // Threaded (skip-pointer) node, one table per traversal order: the six ray-direction classes
 // (+X,-X,+Y,-Y,+Z,-Z) of the multi-threaded BVH, then the single-table threaded BVH in the

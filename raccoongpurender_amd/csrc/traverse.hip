@@ -11,9 +11,9 @@
 // library is built with -ffp-contract=off, so hit index, t, u and v are bit-identical
 // to the oracle on the same tree.
 //
-// Layout (rgpu_types.h): stackless records are 64 B (a leaf or a backtrack step reads
-// only the last 16 B), threaded records are 32 B in one pre-ordered table per ray
-// direction class, primitives are 48 B records in leaf order.
+// Layout (rgpu_types.h): stackless walk records are 128 B, one per two tree levels (a leaf needs
+// none), threaded records are 32 B in one pre-ordered table per ray direction class, primitives
+// are 48 B records in leaf order.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -58,13 +58,13 @@ __device__ __forceinline__ void flush_counts(unsigned long long* counters, const
 }
 
 // One thread per ray, in three forms of the same walk (same visits, same results): plain, the
-// walk as one loop (best for coherent rays, whose lanes reach leaves together anyway); count,
-// the same with event counters; batched, leaves batched across the wave (better for incoherent
-// rays, chosen by a leaf_batch above 1).
+// walk as one loop; count, the same with event counters; batched, leaves batched across the wave
+// (chosen by a leaf_batch above 1). The stackless walk's plain and counting forms are its batched
+// loop with leaf_batch 1.
 enum { kWalkPlain = 0, kWalkCount = 1, kWalkBatched = 2 };
 
-template <int kMode>
-__global__ void __launch_bounds__(256) k_trace_stackless(const TraceRay* __restrict__ rays,
+template <bool kCount>
+__global__ void __launch_bounds__(256, 8) k_trace_stackless(const TraceRay* __restrict__ rays,
                                                          TraceHit* __restrict__ hits, uint32_t n, TraceScene sc,
                                                          uint32_t leaf_batch, unsigned long long* counters) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -74,13 +74,11 @@ __global__ void __launch_bounds__(256) k_trace_stackless(const TraceRay* __restr
         float t;
         load_ray(rays, i, &ro, &rd, &t);
         float u, v;
-        int32_t prim = kMode == kWalkBatched ? trace_batched<kVariantStackless>(sc, ro, rd, &t, &u, &v, leaf_batch)
-                                         : trace_stackless<kMode == kWalkCount>(sc.sl_nodes, sc.prims, sc.sphere_begin,
-                                                                             sc.boxes_finite != 0, ro, rd, &t, &u,
-                                                                             &v, &c);
+        const int32_t prim =
+            trace_batched<kVariantStackless, false, kCount>(sc, ro, rd, &t, &u, &v, leaf_batch, 0, &c);
         store_hit(hits, i, prim, t, u, v);
     }
-    if (kMode == kWalkCount) flush_counts(counters, c);
+    if (kCount) flush_counts(counters, c);
 }
 
 // kVariant: kVariantThreaded (a table per direction class) or kVariantSingleThreaded.
@@ -108,73 +106,74 @@ __global__ void __launch_bounds__(256) k_trace_threaded(const TraceRay* __restri
 // Persistent wave64 traversal: wave w owns rays [w * chunk, (w + 1) * chunk) and hands them to
 // its lanes as lanes finish, refilling whenever at least `refill` lanes are idle (all at once
 // when the wave is idle), so that lanes do not wait for the slowest ray of the wave. No
-// atomics: a wave's cursor is wave-uniform.
+// atomics: a wave's cursor is wave-uniform. A finished ray's hit is stored when its lane takes
+// the next ray (or at the end), with the other finished lanes.
 // Leaves are batched: a lane that enters a leaf stops there, and the wave tests primitives only
 // once `leaf_batch` lanes wait at leaves or at least as many lanes wait as walk on, so that the
 // primitive tests run with many lanes at once instead of taxing every node visit of the wave. Each ray still
 // visits its nodes and tests its primitives in the order of the one-ray walk.
-// Stackless: the first `top` node records (the top of the tree, numbered breadth-first) are
-// copied to LDS at the start (top * 64 bytes of dynamic shared memory) and read from there.
+// Stackless: the first `top` walk records (the top of the tree, numbered breadth-first) are
+// copied to LDS at the start and read from there (walk_lds: the records, then the stacks).
 template <int kVariant>
-__global__ void __launch_bounds__(256) k_trace_persistent(const TraceRay* __restrict__ rays,
+__global__ void __launch_bounds__(256, kVariant == kVariantStackless ? 7 : 1) k_trace_persistent(const TraceRay* __restrict__ rays,
                                                           TraceHit* __restrict__ hits, uint32_t n, TraceScene sc,
                                                           uint32_t chunk, uint32_t refill, uint32_t leaf_batch,
                                                           uint32_t top) {
-    const SLTreelet src{reinterpret_cast<const float4*>(sc.sl_nodes), top};
-    if constexpr (kVariant == kVariantStackless) {
-        for (uint32_t j = threadIdx.x; j < 4 * top; j += blockDim.x) sl_treelet[j] = src.g[j];
-        __syncthreads();
-    }
+    constexpr bool kStackless = kVariant == kVariantStackless;
+    uint32_t spill[kStackless ? kWalkStackSpill : 1];
+    const WalkStack stk = walk_stack(top, spill);
+    const float4* recs = reinterpret_cast<const float4*>(sc.walk_nodes);
+    if constexpr (kStackless) stage_records(recs, top);
     const uint32_t lane = threadIdx.x & 63;
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    // the wave's cursor in scalar registers, so that the loop's control costs no vector operations
+    const uint32_t wave = (uint32_t)wave_scalar((int32_t)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
     const unsigned long long below = (1ull << lane) - 1ull;
     uint64_t next = (uint64_t)wave * chunk;
     const uint64_t end = next + chunk < (uint64_t)n ? next + chunk : (uint64_t)n;
     uint32_t ray = kInvalid;
-    using State = typename std::conditional<kVariant == kVariantStackless, StacklessRay, ThreadedRay>::type;
+    using State = typename std::conditional<kStackless, StacklessRay, ThreadedRay>::type;
     State st;
     st.node = kInvalid;
-    if constexpr (kVariant != kVariantStackless) st.leaf = 0;
+    if constexpr (!kStackless) st.leaf = 0;
     const bool finite = sc.boxes_finite != 0;
+    int32_t kind = 0;  // a scalar: how the live rays may visit records
     for (;;) {
-        const bool idle = !walk_live(st);
-        const unsigned long long idle_mask = __ballot(idle);
-        const uint32_t nidle = (uint32_t)__popcll(idle_mask);
-        if (nidle >= refill || nidle == 64u) {
+        uint32_t nwalk = count_lanes(walk_walking(st)), npending = count_lanes(walk_pending(st));
+        const uint32_t nidle = 64u - nwalk - npending;
+        if (next < end ? (nidle >= refill || nidle == 64u) : nidle == 64u) {
+            const bool idle = !walk_live(st);
+            const unsigned long long idle_mask = __ballot(idle);
             if (idle) {
+                if (ray != kInvalid) store_hit(hits, ray, st.prim, st.tmin, st.u, st.v);
+                ray = kInvalid;
                 const uint64_t r = next + (uint64_t)__popcll(idle_mask & below);
                 if (r < end) {
                     ray = (uint32_t)r;
                     F3 ro, rd;
                     float tmax;
                     load_ray(rays, ray, &ro, &rd, &tmax);
-                    if constexpr (kVariant != kVariantStackless)
-                        threaded_begin<kVariant>(st, sc.mt_nodes, sc.nnodes, ro, rd, tmax);
-                    else
-                        stackless_begin(st, ro, rd, tmax);
+                    if constexpr (kStackless) stackless_begin(st, stk, sc.root, ro, rd, tmax);
+                    else threaded_begin<kVariant>(st, sc.mt_nodes, sc.nnodes, ro, rd, tmax);
                 }
             }
+            if (next >= end) break;  // every lane was idle and nothing is left to hand out
             next += nidle;
+            if constexpr (kStackless) kind = visit_kind(st, finite);
+            nwalk = count_lanes(walk_walking(st));
+            npending = count_lanes(walk_pending(st));
         }
-        if (__ballot(walk_live(st)) == 0) break;
-        const bool pending = walk_pending(st);
-        const bool walking = walk_live(st) && !pending;
-        const uint32_t npending = (uint32_t)__popcll(__ballot(pending));
-        const uint32_t nwalk = (uint32_t)__popcll(__ballot(walking));
-        const bool leaf_phase = npending >= leaf_batch || npending >= nwalk;
-        if (leaf_phase ? pending : walking) {
-            if (leaf_phase) {
-                if constexpr (kVariant != kVariantStackless)
-                    threaded_leaf(st, sc.prims, sc.sphere_begin);
-                else
-                    stackless_leaf(st, src, sc.prims, sc.sphere_begin);
-            } else {
-                if constexpr (kVariant != kVariantStackless)
-                    threaded_visit(st, finite);
-                else
-                    stackless_visit(st, src, finite);
+        if (npending >= leaf_batch || npending >= nwalk) {
+            if (walk_pending(st)) {
+                if constexpr (kStackless) stackless_leaf<false>(st, stk, sc.prims, sc.sphere_begin, nullptr);
+                else threaded_leaf(st, sc.prims, sc.sphere_begin);
             }
-            if (!walk_live(st)) store_hit(hits, ray, st.prim, st.tmin, st.u, st.v);
+            if constexpr (kStackless) kind = visit_kind_after(kind, st);
+        } else if (walk_walking(st)) {
+            if constexpr (kStackless) {
+                stackless_visit_as<true, false>(kind, st, stk, recs, top, nullptr);
+            } else {
+                threaded_visit(st, finite);
+            }
         }
     }
 }
@@ -210,9 +209,12 @@ hipError_t launch_trace(const TraceScene& sc, int variant, const TraceRay* rays,
     if (block == 0 && !counters && sc.nnodes != 0) {
         // persistent kernel: as many resident waves as fit, each with a chunk of the rays
         const uint32_t cus = tune && tune->cu_count ? tune->cu_count : 256u;
-        const uint32_t wps = tune && tune->waves_per_simd ? tune->waves_per_simd : 8u;
-        // measured on the 1.3M-triangle incoherent set: refills at 24 (stackless) or 48 (threaded)
-        // idle lanes, primitive tests once 8 (stackless) or 6 (threaded) lanes wait at leaves
+        // measured on the 1.3M-triangle incoherent set: 7 (stackless) or 8 (threaded) waves per SIMD,
+        // refills at 24 or 48 idle lanes, primitive tests once 12 or 6 lanes wait at leaves. The
+        // stackless walk at 8 waves fetches more from beyond the L2 and is slower: 0.88 ms against
+        // 0.77 (6 waves 0.81)
+        const uint32_t wps = tune && tune->waves_per_simd ? tune->waves_per_simd
+                             : variant == kVariantStackless ? kDefaultWavesStackless : 8u;
         const uint32_t refill =
             tune && tune->refill ? tune->refill : (variant != kVariantStackless ? 48u : 24u);
         const uint32_t leaf_batch = tune && tune->leaf_batch ? tune->leaf_batch
@@ -228,13 +230,13 @@ hipError_t launch_trace(const TraceScene& sc, int variant, const TraceRay* rays,
             hipLaunchKernelGGL(k_trace_persistent<kVariantSingleThreaded>, dim3(blocks), dim3(256), 0, stream, rays,
                                hits, n, sc, chunk, refill, leaf_batch, 0u);
         } else {
-            // the top of the tree in LDS: 320 records (20 KB) let the 8 workgroups per CU of the
-            // default launch share the CU's 160 KB
+            // the top of the tree in LDS: 128 records (14 KB) beside 8 KB of stacks let the 7
+            // workgroups per CU of the default launch share the CU's 160 KB
             uint32_t top = tune && tune->treelet ? tune->treelet : kDefaultTreelet;
             if (top == kTreeletOff) top = 0;
-            top = top < sc.nnodes ? top : sc.nnodes;
-            top = top < kTreeletMaxNodes ? top : kTreeletMaxNodes;
-            hipLaunchKernelGGL(k_trace_persistent<kVariantStackless>, dim3(blocks), dim3(256), (size_t)top * 64u,
+            top = top < sc.nwalk ? top : sc.nwalk;
+            top = top < kTreeletMaxStaged ? top : kTreeletMaxStaged;
+            hipLaunchKernelGGL(k_trace_persistent<kVariantStackless>, dim3(blocks), dim3(256), walk_lds_bytes(top, 256),
                                stream, rays, hits, n, sc, chunk, refill, leaf_batch, top);
         }
         return hipGetLastError();
@@ -252,15 +254,12 @@ hipError_t launch_trace(const TraceScene& sc, int variant, const TraceRay* rays,
     } else if (variant == kVariantSingleThreaded) {
         launch_threaded<kVariantSingleThreaded>(mode, grid, block, stream, rays, hits, n, sc, leaf_batch, counters);
     } else {
+        const size_t lds = walk_lds_bytes(0, block);
         if (mode == kWalkCount)
-            hipLaunchKernelGGL(k_trace_stackless<kWalkCount>, grid, dim3(block), 0, stream, rays, hits, n, sc,
-                               leaf_batch, counters);
-        else if (mode == kWalkBatched)
-            hipLaunchKernelGGL(k_trace_stackless<kWalkBatched>, grid, dim3(block), 0, stream, rays, hits, n, sc,
-                               leaf_batch, counters);
+            hipLaunchKernelGGL(k_trace_stackless<true>, grid, dim3(block), lds, stream, rays, hits, n, sc, 1u, counters);
         else
-            hipLaunchKernelGGL(k_trace_stackless<kWalkPlain>, grid, dim3(block), 0, stream, rays, hits, n, sc,
-                               leaf_batch, counters);
+            hipLaunchKernelGGL(k_trace_stackless<false>, grid, dim3(block), lds, stream, rays, hits, n, sc, leaf_batch,
+                               counters);
     }
     return hipGetLastError();
 }

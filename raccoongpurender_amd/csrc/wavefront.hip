@@ -942,17 +942,15 @@ __device__ __forceinline__ void store_extension(const DevState& s, const TraceSc
 // extension_ray_cast (kernels/extension_ray_cast_stackless.cl:202-246) over every slot, one
 // thread per slot.
 template <int kVariant, class J>
-__global__ void __launch_bounds__(256) k_trace_step(DevState s, WFParams p, J jobs, uint32_t top) {
+__global__ void __launch_bounds__(256, 8) k_trace_step(DevState s, WFParams p, J jobs, uint32_t top) {
     const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
     if constexpr (kVariant == kVariantStackless) {
         // the top `top` records of the block's scene in LDS (a job owns whole 256-slot blocks,
         // so every slot of a workgroup traces the same scene)
         const uint32_t first = blockIdx.x * blockDim.x;
         const TraceScene sb = jobs.scene(jobs.job(first < p.n ? first : p.n - 1));
-        const uint32_t t = top < sb.nnodes ? top : sb.nnodes;
-        const float4* g = reinterpret_cast<const float4*>(sb.sl_nodes);
-        for (uint32_t j = threadIdx.x; j < 4 * t; j += blockDim.x) sl_treelet[j] = g[j];
-        __syncthreads();
+        const uint32_t t = top < sb.nwalk ? top : sb.nwalk;
+        stage_records(reinterpret_cast<const float4*>(sb.walk_nodes), t);
         top = t;
     }
     advance_cursors(s, jobs, slot);
@@ -1527,9 +1525,10 @@ hipError_t step_impl(const DevState& st, const WFParams& p, const J& jobs, const
     } else if (variant == kVariantSingleThreaded) {
         hipLaunchKernelGGL((k_trace_step<kVariantSingleThreaded, J>), tgrid, tblk, 0, s, st, p, jobs, 0u);
     } else {
-        // the top of the tree in LDS: 80 records per wave, so that 8 waves per SIMD fit the 160 KB
-        const uint32_t top = kDefaultTreelet * tb / 256u;
-        hipLaunchKernelGGL((k_trace_step<kVariantStackless, J>), tgrid, tblk, (size_t)top * 64u, s, st, p, jobs,
+        // the top of the tree in LDS: 27 records per wave beside its 2 KB of stacks, so that 8 waves
+        // per SIMD fit the 160 KB
+        const uint32_t top = 27u * tb / 64u;
+        hipLaunchKernelGGL((k_trace_step<kVariantStackless, J>), tgrid, tblk, walk_lds_bytes(top, tb), s, st, p, jobs,
                            top);
     }
     mark(7);

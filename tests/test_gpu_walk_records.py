@@ -1,0 +1,82 @@
+"""The stackless walk's record form: deep stacks, rays without motion along an axis, odd clips.
+
+Bit-exact against the oracle's binary walk on the same tree, as the other traversal tests: the
+walk takes two tree levels a visit, keeps what it defers in LDS and then in private memory, and
+visits binary nodes one by one where a wave's rays allow nothing else.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+from raccoongpurender_amd import _lib, scenes
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+SAME = dict(prim=0, t=0, uv=0)
+
+
+def _check(ctx, v, f, rays, sph=None, **opt):
+    bvh = _lib.BVH(v, f, sph, **opt)
+    scene = _lib.Scene(ctx, bvh)
+    o, _ = O.intersect_stackless(O.RefStackless(bvh.export()), v, f, rays, sph)
+    for block in (0, 64, 256):
+        g = _lib.trace(ctx, scene, rays, "stackless", block=block)
+        assert H.compare_hits(g, o) == SAME, (block, bvh.depth)
+    scene.close()
+    return bvh
+
+
+def _facing_triangles(x, size):
+    """One triangle per x, in the plane of that x, around the x axis."""
+    corner = np.array([[-1.0, -1.0], [2.5, -1.0], [-1.0, 2.5]])
+    v = np.zeros((len(x), 3, 3))
+    v[:, :, 0] = x[:, None]
+    v[:, :, 1:] = corner[None] * size[:, None, None]
+    return v.reshape(-1, 3).astype(np.float32), np.arange(3 * len(x), dtype=np.uint32).reshape(-1, 3)
+
+
+@pytest.mark.parametrize("bins", (2, 16))
+def test_chains_deeper_than_the_lds_stack(ctx, bins):
+    # triangles that double in size and distance split off one by one: rays from the small end
+    # defer a leaf on every level of a chain far longer than the stack's eight LDS entries
+    k = np.arange(56)
+    v, f = _facing_triangles(2.0 ** -k, 0.5 * 2.0 ** -k)
+    rng = np.random.default_rng(3)
+    n = 4096
+    ro = np.stack([np.full(n, -1e-3), *(rng.normal(size=(2, n)) * 2.0 ** rng.uniform(-50, 0, (2, n)))], 1)
+    rd = np.stack([np.ones(n), *(rng.normal(size=(2, n)) * 1e-3)], 1)
+    rd[::5, 1] = 0.0  # and without motion along an axis
+    bvh = _check(ctx, v, f, scenes.make_rays(ro, rd), max_leaf=1, bins=bins)
+    assert bvh.depth > 16
+
+
+def test_balanced_stack_past_the_lds_entries(ctx):
+    # coincident spheres: every box is every other, each ray defers on all 13 levels
+    sph = np.tile(np.array([[0.0, 0.0, 0.0, 1.0]], np.float32), (5000, 1))
+    rays = scenes.incoherent_rays(300, [-2, -2, -2], [2, 2, 2], seed=5)
+    v, f = np.zeros((0, 3), np.float32), np.zeros((0, 3), np.uint32)
+    assert _check(ctx, v, f, rays, sph, max_leaf=1).depth >= 13
+
+
+@pytest.mark.parametrize("mesh", ("grid", "icosphere", "soup"))
+def test_axis_aligned_and_clipped_rays(ctx, mesh):
+    # zero direction components (of either sign) with origins on and off the boxes' planes, far
+    # clips of every kind, and all of them mixed into the waves
+    v, f = {"grid": lambda: H.grid_plane(24), "icosphere": lambda: scenes.displaced_icosphere(level=4),
+            "soup": lambda: H.triangle_soup(3000, 6)}[mesh]()
+    lo, hi = v.min(0), v.max(0)
+    rng = np.random.default_rng(7)
+    n = 6000
+    ro = np.where(rng.random((n, 1)) < 0.5, v[rng.integers(0, len(v), n)], lo + (hi - lo) * rng.random((n, 3)))
+    rd = rng.normal(size=(n, 3))
+    zero = rng.integers(0, 8, n)  # which components are zero; 7 leaves no motion at all
+    for a in range(3):
+        rd[(zero >> a) & 1 == 1, a] = rng.choice([0.0, -0.0])
+    ro[:, :] -= (rng.random((n, 1)) < 0.5) * rd * 3.0
+    rays = scenes.make_rays(ro, rd)
+    only_flat = rays[(zero > 0) & (zero < 7)]
+    _check(ctx, v, f, only_flat)
+    rays["tmax"][::3] = rng.choice([0.0, -1.0, 0.5, np.inf, np.nan], len(rays[::3])).astype(np.float32)
+    rays["ro"][5::41, 0] = np.inf
+    _check(ctx, v, f, rays)
