@@ -141,18 +141,17 @@ int rgpu_bvh_export(const rgpu_bvh* bvh, float* bounds, int32_t* left, int32_t* 
 
 /* ---------------------------------------------------------------- scene (device)
  * Replaces SceneManager::createBuffer (common/scene_manager.hpp:579-591) and the
- * SceneBuffer it fills (common/scene_manager.hpp:284-294): packs the stackless walk
- * records, the threaded node tables (one per ray-direction class and one for the single-table
- * walk, each in its own pre-order) and the primitive records, and uploads them with the
- * vertices. Host arrays are copied; the caller keeps ownership. A BVH of 2^30 nodes or more
+ * SceneBuffer it fills (common/scene_manager.hpp:284-294): packs the walk records (every
+ * traversal variant reads them; the threaded variants' child orders are bits in them) and the
+ * primitive records, and uploads them with the vertices. Host arrays are copied; the caller keeps ownership. A BVH of 2^30 nodes or more
  * (over 2^29 primitives) is refused with RGPU_ERR_INVALID_ARG: the walk's node ids carry two
  * flag bits. */
 int rgpu_scene_create(rgpu_ctx* ctx, const rgpu_bvh* bvh, const float* points, uint32_t stride, uint32_t npoints,
                       const uint32_t* indices, uint32_t ntris, const float* spheres, uint32_t nspheres,
                       rgpu_scene** out);
 int rgpu_scene_destroy(rgpu_scene* scene);
-/* Device bytes held by the scene per table: [stackless nodes, the seven threaded tables,
- * primitive records, vertices]. */
+/* Device bytes held by the scene per table: [walk records, 0 (the threaded variants have no tables
+ * of their own), primitive records, vertices]. */
 int rgpu_scene_bytes(const rgpu_scene* scene, uint64_t* out4);
 
 /* ---------------------------------------------------------------- extension ray cast
@@ -168,14 +167,12 @@ int rgpu_extension_ray_cast(rgpu_ctx* ctx, rgpu_stream stream, const rgpu_scene*
 /* Launch shape of the persistent ray-cast kernel used when block == 0: resident waves per
  * SIMD (grid = CUs * waves_per_simd workgroups of 256; 1..16), the number of idle lanes of a
  * wave that makes it hand out its next rays (1..64), and the number of lanes waiting at leaves
- * that makes it test their primitives (1..64). 0 keeps the default (7 waves for stackless, 8 for
- * threaded; refill at 24 idle lanes for stackless, 48 for threaded; leaves at 12 waiting lanes for
- * stackless, 6 for threaded, or once as many lanes wait as walk on). leaf_batch also applies to
- * the one-thread-per-ray kernels (block != 0), whose
- * default is 64 (leaves only once as many lanes wait as walk on) and where 1 selects the plain
- * one-ray walk. treelet: the number of top-of-tree stackless walk records each
- * workgroup of the persistent kernel copies to LDS and reads from there (1..1024, 112 bytes
- * each, as many as fit; 0 = default 128; RGPU_TREELET_OFF = none). Results do not depend on any of them. No
+ * that makes it test their primitives (1..64). 0 keeps the default (7 waves; refill at 24 idle
+ * lanes; leaves at 12 waiting lanes, or once as many lanes wait as walk on). leaf_batch also
+ * applies to the one-thread-per-ray kernels (block != 0), whose default is 64 (leaves only once as
+ * many lanes wait as walk on). treelet: the number of top-of-tree walk records each workgroup of
+ * the persistent kernel copies to LDS and reads from there (1..1024, 112 bytes each, as many as
+ * fit; 0 = default 128; RGPU_TREELET_OFF = none). Results do not depend on any of them. No
  * counterpart in the reference (it leaves launch shapes to the OpenCL driver,
  * common/raccoon_ocl.hpp:906). */
 #define RGPU_TREELET_OFF 0xFFFFFFFFu

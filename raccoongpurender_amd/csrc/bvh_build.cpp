@@ -412,9 +412,31 @@ uint32_t pack_walk(const BVHTree& t, uint32_t top, std::vector<WalkNode>* out) {
             id[i] = (uint32_t)order.size();
             order.push_back((int32_t)i);
         }
+    // Whether a branch's right child comes first, a bit per direction class. The six direction
+    // sorts are applied one after another to the same tree, as common/threaded_bvh.hpp:518-525
+    // does, so a child pair whose centres tie is swapped by every sort.
+    auto orders = [&](int32_t i) {
+        uint32_t bits = 0;
+        bool swapped = false;
+        for (int dir = 0; branch(i) && dir < 6; ++dir) {
+            const BuildNode& a = nodes[swapped ? nodes[i].right : nodes[i].left];
+            const BuildNode& b = nodes[swapped ? nodes[i].left : nodes[i].right];
+            const int axis = dir / 2;
+            float lc = 0.5f * (a.bmin[axis] + a.bmax[axis]);
+            float rc = 0.5f * (b.bmin[axis] + b.bmax[axis]);
+            if (dir & 1) std::swap(lc, rc);
+            if (!(lc < rc)) swapped = !swapped;
+            bits |= (swapped ? 1u : 0u) << dir;
+        }
+        return bits;
+    };
     out->resize(order.size());
     for (size_t r = 0; r < order.size(); ++r) {
         WalkNode& w = (*out)[r];
+        const uint32_t o[3] = {orders(order[r]), orders(nodes[order[r]].left), orders(nodes[order[r]].right)};
+        w.order = 0;
+        for (int dir = 0; dir < 6; ++dir)
+            for (int k = 0; k < 3; ++k) w.order |= ((o[k] >> dir) & 1u) << (3 * dir + k);
         int32_t g[4];
         family(order[r], g);
         for (int k = 0; k < 4; ++k) {
@@ -423,72 +445,12 @@ uint32_t pack_walk(const BVHTree& t, uint32_t top, std::vector<WalkNode>* out) {
                 w.box[k][3 + a] = nodes[g[k]].bmax[a];
             }
             w.link[k] = branch(g[k]) ? 8 * id[g[k]] : word(g[k]);
-            w.pad[k] = 0;
         }
+        for (uint32_t& x : w.pad) x = 0;
         for (int k = 0; k < 4; k += 2)
             if (g[k] == g[k + 1]) w.link[k + 1] = kInvalid;  // a leaf child
     }
     return 0;
-}
-
-void pack_threaded(const BVHTree& t, std::vector<MTNode>* out) {
-    const uint32_t nn = (uint32_t)t.nodes.size();
-    out->assign((size_t)kMTOrders * nn, MTNode());
-    if (nn == 0) return;
-    // Mutable child order; the six direction sorts are applied one after another to
-    // the same tree, as common/threaded_bvh.hpp:518-525 does, so a child pair whose
-    // centres tie is swapped by every sort. The single table keeps the build's order.
-    std::vector<int32_t> L(nn), R(nn);
-    for (uint32_t i = 0; i < nn; ++i) {
-        L[i] = t.nodes[i].left;
-        R[i] = t.nodes[i].right;
-    }
-    std::vector<uint32_t> size(nn, 1);
-    for (int32_t i = (int32_t)nn - 1; i >= 0; --i)
-        if (L[i] >= 0) size[i] = 1 + size[L[i]] + size[R[i]];
-    std::vector<std::pair<uint32_t, uint32_t>> stack;  // (node, position in this direction's order)
-    for (int dir = 0; dir < kMTOrders; ++dir) {
-        if (dir < 6) {
-            const int axis = dir / 2;
-            const bool negative = (dir & 1) != 0;
-            for (uint32_t i = 0; i < nn; ++i) {
-                if (L[i] < 0) continue;
-                const BuildNode& a = t.nodes[L[i]];
-                const BuildNode& b = t.nodes[R[i]];
-                float lc = 0.5f * (a.bmin[axis] + a.bmax[axis]);
-                float rc = 0.5f * (b.bmin[axis] + b.bmax[axis]);
-                if (negative) std::swap(lc, rc);
-                if (!(lc < rc)) std::swap(L[i], R[i]);
-            }
-        } else {
-            for (uint32_t i = 0; i < nn; ++i) {
-                L[i] = t.nodes[i].left;
-                R[i] = t.nodes[i].right;
-            }
-        }
-        MTNode* tab = out->data() + (size_t)dir * nn;
-        stack.clear();
-        stack.push_back({0u, 0u});
-        while (!stack.empty()) {
-            auto [node, pos] = stack.back();
-            stack.pop_back();
-            const BuildNode& b = t.nodes[node];
-            MTNode& m = tab[pos];
-            for (int k = 0; k < 3; ++k) {
-                m.bmin[k] = b.bmin[k];
-                m.bmax[k] = b.bmax[k];
-            }
-            uint32_t next = pos + size[node];
-            m.miss = next < nn ? next : kInvalid;
-            if (L[node] >= 0) {
-                m.leaf = 0;
-                stack.push_back({(uint32_t)R[node], pos + 1 + size[L[node]]});
-                stack.push_back({(uint32_t)L[node], pos + 1});
-            } else {
-                m.leaf = kLeafFlag | ((b.prim_cnt - 1) << 28) | b.prim_beg;
-            }
-        }
-    }
 }
 
 void pack_prims(const BVHTree& t, const float* points, uint32_t stride,

@@ -49,13 +49,10 @@ void pack_stackless(const BVHTree& t, std::vector<SLNode>* out);
 void number_top_breadth_first(std::vector<SLNode>* nodes, uint32_t top);
 // Sets kChildLeaf on the child and sibling ids that name leaves (after any renumbering).
 void mark_leaf_links(std::vector<SLNode>* nodes);
-// Records of the device's stackless walk: the first `top` in breadth-first order (so that any LDS
+// Records of the device's walk: the first `top` in breadth-first order (so that any LDS
 // copy of the top of the tree is a prefix), the others in the tree's depth-first order. Returns
 // the root's link.
 uint32_t pack_walk(const BVHTree& t, uint32_t top, std::vector<WalkNode>* out);
-// out: kMTOrders tables of t.nodes.size() records, order-major (+X,-X,+Y,-Y,+Z,-Z, then the
-// single table in the build's child order).
-void pack_threaded(const BVHTree& t, std::vector<MTNode>* out);
 void pack_prims(const BVHTree& t, const float* points, uint32_t stride,
                 const uint32_t* indices, uint32_t ntris,
                 const float* spheres, uint32_t nspheres, std::vector<PrimRec>* out);

@@ -334,7 +334,7 @@ static int upload_new(rgpu_ctx* ctx, const void* src, size_t bytes, void** dst) 
 int rgpu_scene_destroy(rgpu_scene* s) {
     if (!s) return RGPU_ERR_INVALID_ARG;
     if (s->ctx) (void)hipSetDevice(s->ctx->device);
-    for (void* p : {s->sl, s->mt, s->prims, s->points, s->indices, s->spheres})
+    for (void* p : {s->walk, s->prims, s->points, s->indices, s->spheres})
         if (p) (void)hipFree(p);
     delete s;
     return RGPU_OK;
@@ -354,7 +354,6 @@ int rgpu_scene_create(rgpu_ctx* ctx, const rgpu_bvh* bvh, const float* points, u
     RGPU_GUARD_BEGIN
     RGPU_HIP(ctx, hipSetDevice(ctx->device));
     std::vector<SLNode> sl;
-    std::vector<MTNode> mt;
     std::vector<PrimRec> pr;
     std::vector<WalkNode> walk;
     // beside the other packers (its future waits for it on every way out)
@@ -364,7 +363,6 @@ int rgpu_scene_create(rgpu_ctx* ctx, const rgpu_bvh* bvh, const float* points, u
     number_top_breadth_first(&sl, kTreeletMaxNodes);
     mark_leaf_links(&sl);
     const uint64_t sl_print = fingerprint64(sl.data(), sl.size() * sizeof(SLNode), ntris);
-    pack_threaded(bvh->tree, &mt);
     pack_prims(bvh->tree, points, stride, indices, ntris, spheres, nspheres, &pr);
     std::vector<float> p4((size_t)npoints * 4, 0.0f);
     for (uint32_t i = 0; i < npoints; ++i)
@@ -373,8 +371,7 @@ int rgpu_scene_create(rgpu_ctx* ctx, const rgpu_bvh* bvh, const float* points, u
     rgpu_scene* s = new rgpu_scene();
     s->ctx = ctx;
     int rc = RGPU_OK;
-    if (rc == RGPU_OK) rc = upload_new(ctx, walk.data(), walk.size() * sizeof(WalkNode), &s->sl);
-    if (rc == RGPU_OK) rc = upload_new(ctx, mt.data(), mt.size() * sizeof(MTNode), &s->mt);
+    if (rc == RGPU_OK) rc = upload_new(ctx, walk.data(), walk.size() * sizeof(WalkNode), &s->walk);
     if (rc == RGPU_OK) rc = upload_new(ctx, pr.data(), pr.size() * sizeof(PrimRec), &s->prims);
     if (rc == RGPU_OK) rc = upload_new(ctx, p4.data(), p4.size() * sizeof(float), &s->points);
     if (rc == RGPU_OK) rc = upload_new(ctx, indices, (size_t)ntris * 3 * sizeof(uint32_t), &s->indices);
@@ -383,9 +380,8 @@ int rgpu_scene_create(rgpu_ctx* ctx, const rgpu_bvh* bvh, const float* points, u
         rgpu_scene_destroy(s);
         return rc;
     }
-    s->dev.walk_nodes = (const WalkNode*)s->sl;
+    s->dev.walk_nodes = (const WalkNode*)s->walk;
     s->dev.nwalk = (uint32_t)walk.size();
-    s->dev.mt_nodes = (const MTNode*)s->mt;
     s->dev.prims = (const PrimRec*)s->prims;
     s->dev.points = (const float4*)s->points;
     s->dev.indices = (const uint32_t*)s->indices;
@@ -402,11 +398,11 @@ int rgpu_scene_create(rgpu_ctx* ctx, const rgpu_bvh* bvh, const float* points, u
     s->fingerprint = fingerprint64(pr.data(), pr.size() * sizeof(PrimRec), sl_print);
     if (!bvh->tree.nodes.empty())
         for (int k = 0; k < 3; ++k) {
-            s->lo[k] = bvh->tree.nodes[0].bmin[k];
-            s->hi[k] = bvh->tree.nodes[0].bmax[k];
+            s->lo[k] = s->dev.root_lo[k] = bvh->tree.nodes[0].bmin[k];
+            s->hi[k] = s->dev.root_hi[k] = bvh->tree.nodes[0].bmax[k];
         }
     s->bytes[0] = walk.size() * sizeof(WalkNode);
-    s->bytes[1] = mt.size() * sizeof(MTNode);
+    s->bytes[1] = 0;  // the threaded walks' child orders are bits of the walk records
     s->bytes[2] = pr.size() * sizeof(PrimRec);
     s->bytes[3] = p4.size() * sizeof(float) + (size_t)ntris * 12 + (size_t)nspheres * 16;
     *out = s;

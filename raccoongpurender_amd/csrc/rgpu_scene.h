@@ -8,8 +8,7 @@
 struct rgpu_scene {
     rgpu_ctx* ctx = nullptr;
     rgpu::TraceScene dev;
-    void* sl = nullptr;
-    void* mt = nullptr;
+    void* walk = nullptr;
     void* prims = nullptr;
     void* points = nullptr;
     void* indices = nullptr;

@@ -22,16 +22,16 @@ struct alignas(16) TraceHit {
     float v;
 };
 
-// kVariantThreaded: the multi-threaded BVH (a link table per ray-direction class);
-// kVariantSingleThreaded: the single-table threaded BVH. Both walk the same box records.
+// kVariantThreaded: the multi-threaded BVH (a child order per ray-direction class);
+// kVariantSingleThreaded: the threaded BVH in the build's own child order. All walk the same records.
 enum { kVariantStackless = 0, kVariantThreaded = 1, kVariantSingleThreaded = 2 };
 
 // Device-resident scene as the kernels see it.
 struct TraceScene {
-    const WalkNode* walk_nodes = nullptr;  // the stackless walk's records
+    const WalkNode* walk_nodes = nullptr;
     uint32_t nwalk = 0;
     uint32_t root = 0;  // the root's walk link: its record, or the word of a root leaf
-    const MTNode* mt_nodes = nullptr;  // kMTOrders tables of nnodes records
+    float root_lo[3] = {0.0f, 0.0f, 0.0f}, root_hi[3] = {0.0f, 0.0f, 0.0f};  // the root's box
     const PrimRec* prims = nullptr;
     const float4* points = nullptr;    // original vertices (for geometric normals)
     const uint32_t* indices = nullptr;  // 3 per triangle
@@ -44,18 +44,21 @@ struct TraceScene {
 // Launch shape of the persistent ray-cast kernel: CUs to fill, resident waves per SIMD (grid =
 // cu_count * waves_per_simd workgroups of 256), the idle-lane count that triggers a refill and
 // the count of lanes waiting at leaves that triggers their primitive tests. Zeros take the
-// defaults (256 CUs; 7 waves, refill at 24 lanes and leaves at 12 waiting lanes for the stackless
-// walk, 8, 48 and 6 for the threaded ones), measured on 4M incoherent rays over 1.3M triangles.
+// defaults below (and 256 CUs).
 struct TraceTuning {
     uint32_t cu_count = 0;
     uint32_t waves_per_simd = 0;
     uint32_t refill = 0;
     uint32_t leaf_batch = 0;
-    uint32_t treelet = 0;  // stackless records staged in LDS per workgroup; kTreeletOff: none
+    uint32_t treelet = 0;  // walk records staged in LDS per workgroup; kTreeletOff: none
 };
-constexpr uint32_t kDefaultLeafBatch = 6;
-constexpr uint32_t kDefaultLeafBatchStackless = 12;
-constexpr uint32_t kDefaultWavesStackless = 7;
+// Measured on 4.19 M incoherent rays over 1.3M triangles, stackless: 7 waves per SIMD 0.77 ms (8:
+// 0.88, more traffic from beyond the L2; 6: 0.81), refills at 24 idle lanes, leaves at 12 waiting
+// lanes (8, 16: 1 % slower), 128 staged records (none: 1.04; 14 KB beside 8 KB of stacks let 7
+// workgroups share a CU's 160 KB).
+constexpr uint32_t kDefaultWaves = 7;
+constexpr uint32_t kDefaultRefill = 24;
+constexpr uint32_t kDefaultLeafBatch = 12;
 // One thread per ray (coherent rays, the wavefront's per-slot trace): leaves wait until as many
 // lanes wait as walk on.
 constexpr uint32_t kPerRayLeafBatch = 64;
@@ -64,17 +67,21 @@ constexpr uint32_t kPerRayLeafBatch = 64;
 constexpr uint32_t kTreeletMaxNodes = 1024;
 constexpr uint32_t kTreeletOff = 0xFFFFFFFFu;
 constexpr uint32_t kDefaultTreelet = 128;
-// Stack entries of a stackless walk in LDS, one column per lane, and behind them in private
-// memory: a walk defers at most one link per level, and leaves lie at depth 64 at most.
+// Stack entries of a walk in LDS, one column per lane, and behind them in private memory: a walk
+// defers at most one link per level, and leaves lie at depth 64 at most.
 constexpr uint32_t kWalkStackLds = 8;
 constexpr uint32_t kWalkStackSpill = 64 - kWalkStackLds;
 constexpr uint32_t kStagedBytes = 112;  // of a walk record in LDS
-// Dynamic LDS of a kernel that walks stackless records: staged records, then the stacks.
-constexpr size_t walk_lds_bytes(uint32_t top, uint32_t threads) {
-    return (size_t)top * kStagedBytes + (size_t)threads * kWalkStackLds * 4u;
+// Bytes of `top` staged records: kVariantThreaded needs their order words too.
+constexpr uint32_t staged_bytes(int variant, uint32_t top) {
+    return top * kStagedBytes + (variant == kVariantThreaded ? (4u * top + 15u) / 16u * 16u : 0u);
+}
+// Dynamic LDS of a kernel that walks: staged records, then the stacks.
+constexpr size_t walk_lds_bytes(int variant, uint32_t top, uint32_t threads) {
+    return (size_t)staged_bytes(variant, top) + (size_t)threads * kWalkStackLds * 4u;
 }
 // (a launch of 256 threads stages at most what 64 KB leave beside the stacks)
-constexpr uint32_t kTreeletMaxStaged = (65536u - 256u * kWalkStackLds * 4u) / kStagedBytes;
+constexpr uint32_t kTreeletMaxStaged = (65536u - 256u * kWalkStackLds * 4u) / (kStagedBytes + 4u);
 
 // counters: null for the production kernels; otherwise 5 device u64 totals
 // {branch visits, leaf visits, parent steps, primitive tests, threaded node visits}.

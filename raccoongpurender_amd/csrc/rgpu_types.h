@@ -41,44 +41,29 @@ static const uint32_t kLeafFlag = 0x80000000u;
 static const uint32_t kChildLeaf = 0x40000000u;
 static const uint32_t kInvalid = 0xFFFFFFFFu;
 
-// Record of the stackless walk on the device, one 128-byte line per branch node at an even depth:
-// the boxes of its four grandchildren (6 floats each, min xyz then max xyz; left child's first)
-// and their links. A link is
+// Record of the walk on the device, one 128-byte line per branch node at an even depth: the boxes
+// of its four grandchildren (6 floats each, min xyz then max xyz; left child's first), their links
+// and the child orders. A link is
 //   a branch's   8 * its record's id (the record's index in 16-byte units); kFirstHalf or
-//                kSecondHalf added means that child of the record's node alone;
+//                kSecondHalf added means that child of the record's node alone, kOneBox + k its
+//                k-th box alone;
 //   a leaf's     kLeafFlag | ((count - 1) << 28) | first slot, its primitive word (never all ones:
 //                first + count <= 2^28 - 1).
 // A child that is a leaf itself fills both of its boxes with its own and has kInvalid for its
 // second link. Record ids stay below 2^28 (a tree has fewer than 2^28 primitives).
+// order: three bits per ray-direction class (+X,-X,+Y,-Y,+Z,-Z, from bit 0) of the multi-threaded
+// BVH (common/threaded_bvh.hpp:494-525): whether the right child comes first, and the same for the
+// left and the right child's children. These 18 bits hold what six pre-ordered node tables held.
 struct alignas(128) WalkNode {
     float box[4][6];
     uint32_t link[4];
-    uint32_t pad[4];
+    uint32_t order;
+    uint32_t pad[3];
 };
 static_assert(sizeof(WalkNode) == 128, "walk record must be one 128-byte line");
 static const uint32_t kFirstHalf = 1;
 static const uint32_t kSecondHalf = 2;
-
-// Threaded (skip-pointer) node, one table per traversal order: the six ray-direction classes
-// (+X,-X,+Y,-Y,+Z,-Z) of the multi-threaded BVH, then the single-table threaded BVH in the
-// build's own child order (common/threaded_bvh.hpp:269-364). Each table is the tree re-laid out
-// in the depth-first pre-order of that order's child ordering (common/threaded_bvh.hpp:494-516
-// for the directions), so the hit link of a branch is always the next record and need not be
-// stored; the miss link is the record that follows the node's subtree
-// (common/threaded_bvh.hpp:417-484, 309-360).
-//   q0 = { bmin.x, bmin.y, bmin.z, bmax.x }
-//   q1 = { bmax.y, bmax.z, miss, leaf }
-// leaf == 0 for a branch; otherwise kLeafFlag | ((count-1) << 28) | first slot.
-// A leaf's hit and miss links are equal (both = miss).
-struct alignas(16) MTNode {
-    float bmin[3];
-    float bmax[3];
-    uint32_t miss;
-    uint32_t leaf;
-};
-static_assert(sizeof(MTNode) == 32, "threaded node record must be 32 bytes");
-constexpr int kMTOrders = 7;  // tables: 6 direction classes, then the single table
-constexpr int kMTSingleOrder = 6;
+static const uint32_t kOneBox = 4;
 
 // Primitive record, one per leaf slot, in leaf order. The triangle edges are the
 // exact float differences v1-v0 and v2-v0 that the Moller-Trumbore test forms

@@ -59,28 +59,6 @@ __device__ __forceinline__ bool plain_slabs(bool boxes_finite, F3 o, F3 inv) {
     return boxes_finite && fo && fi;
 }
 
-template <bool kPlain = false>
-__device__ __forceinline__ bool slab_hit(const float* lo, const float* hi, F3 o, F3 inv, float farclip,
-                                         float* h0, float* h1) {
-    float nx, fx, ny, fy, nz, fz;
-    slab_axis<kPlain>(lo[0], hi[0], o.x, inv.x, &nx, &fx);
-    slab_axis<kPlain>(lo[1], hi[1], o.y, inv.y, &ny, &fy);
-    slab_axis<kPlain>(lo[2], hi[2], o.z, inv.z, &nz, &fz);
-    float rmin = fmaxf(fmaxf(nx, ny), nz);
-    float rmax = fminf(fminf(fx, fy), fz);
-    *h0 = fmaxf(0.0f, rmin);
-    *h1 = fminf(rmax, farclip);
-    return rmin <= rmax && 0.0f <= rmax && rmin <= farclip;
-}
-
-// One box; the wave takes the plain slab form when every active lane may (a wave-uniform branch,
-// so no lane runs both forms).
-__device__ __forceinline__ bool slab_one(const float* lo, const float* hi, F3 o, F3 inv, float farclip, bool plain,
-                                         float* h0, float* h1) {
-    if (__all(plain)) return slab_hit<true>(lo, hi, o, inv, farclip, h0, h1);
-    return slab_hit<false>(lo, hi, o, inv, farclip, h0, h1);
-}
-
 // Test one primitive record; updates (tmin, u, v, prim) when it is the closest so far.
 __device__ __forceinline__ void test_prim(const PrimRec* __restrict__ prims, uint32_t slot, int32_t sphere_begin,
                                           F3 ro, F3 rd, float* tmin, float* uo, float* vo, int32_t* prim) {
@@ -162,134 +140,51 @@ __device__ __forceinline__ uint32_t direction_class(F3 rd) {
     return 0.0f < rd.z ? 4u : 5u;
 }
 
-// The table a ray walks: its direction class for the multi-threaded BVH, the single table
-// otherwise (common/threaded_bvh.hpp:527-547, 366-395).
-template <int kVariant>
-__device__ __forceinline__ const MTNode* threaded_table(const MTNode* tables, uint32_t nnodes, F3 rd) {
-    const uint32_t order = kVariant == kVariantSingleThreaded ? (uint32_t)kMTSingleOrder : direction_class(rd);
-    return tables + (size_t)order * nnodes;
-}
-
-// Threaded traversal of one ray (common/threaded_bvh.hpp:527-569, 366-395).
-template <bool kCount, int kVariant>
-__device__ __forceinline__ int32_t trace_threaded(const MTNode* __restrict__ tables, uint32_t nnodes,
-                                                  const PrimRec* __restrict__ prims, int32_t sphere_begin,
-                                                  bool boxes_finite, F3 ro, F3 rd, float* tmin_io, float* uo,
-                                                  float* vo, Cnt* cnt) {
-    const MTNode* tab = threaded_table<kVariant>(tables, nnodes, rd);
-    const F3 inv = f3(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
-    const bool plain = plain_slabs(boxes_finite, ro, inv);
-    float tmin = *tmin_io;
-    float u = 0.0f, v = 0.0f;
-    int32_t prim = -1;
-    uint32_t node = 0;
-    while (node != kInvalid) {
-        const float4* rec = reinterpret_cast<const float4*>(tab + node);
-        float4 q0 = rec[0], q1 = rec[1];
-        float lo[3] = {q0.x, q0.y, q0.z}, hi[3] = {q0.w, q1.x, q1.y};
-        uint32_t miss = __float_as_uint(q1.z), leaf = __float_as_uint(q1.w);
-        float h0, h1;
-        if (kCount) cnt->node++;
-        bool hit = slab_one(lo, hi, ro, inv, tmin, plain, &h0, &h1);
-        if (hit && leaf != 0) {
-            const uint32_t beg = leaf & 0x0FFFFFFFu;
-            const uint32_t end = beg + ((leaf >> 28) & 7u) + 1u;
-            if (kCount) cnt->prim += end - beg;
-            for (uint32_t s = beg; s < end; ++s) test_prim(prims, s, sphere_begin, ro, rd, &tmin, &u, &v, &prim);
-        }
-        node = (hit && leaf == 0) ? node + 1 : miss;
-    }
-    *tmin_io = tmin;
-    *uo = u;
-    *vo = v;
-    return prim;
-}
-
-// ---------------------------------------------------------------- resumable traversal
-// The same two traversals cut into single steps over explicit per-lane state, so that a lane
-// whose ray has finished can take the next ray while the rest of its wave keeps going. Each
-// ray still visits nodes and tests primitives in exactly the order above.
-
-struct ThreadedRay {
-    const MTNode* tab;
-    F3 ro, rd, inv;
-    float tmin, u, v;
-    int32_t prim;
-    bool plain;     // origin and inverse direction allow the plain slab form (set once per ray)
-    uint32_t node;  // kInvalid when finished
-    uint32_t leaf;  // primitive word of an entered leaf not yet tested (0: none)
-};
-
-template <int kVariant>
-__device__ __forceinline__ void threaded_begin(ThreadedRay& r, const MTNode* tables, uint32_t nnodes, F3 ro, F3 rd,
-                                               float tmax) {
-    r.tab = threaded_table<kVariant>(tables, nnodes, rd);
-    r.ro = ro;
-    r.rd = rd;
-    r.inv = f3(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
-    r.plain = plain_slabs(true, ro, r.inv);
-    r.tmin = tmax;
-    r.u = r.v = 0.0f;
-    r.prim = -1;
-    r.node = 0;
-    r.leaf = 0;
-}
-
-// Box test of the current node of trace_threaded: a branch moves on (hit: next record, miss:
-// miss link); an entered leaf is marked pending with its primitive word kept in r.leaf.
-__device__ __forceinline__ void threaded_visit(ThreadedRay& r, bool boxes_finite) {
-    const float4* rec = reinterpret_cast<const float4*>(r.tab + r.node);
-    float4 q0 = rec[0], q1 = rec[1];
-    float lo[3] = {q0.x, q0.y, q0.z}, hi[3] = {q0.w, q1.x, q1.y};
-    uint32_t miss = __float_as_uint(q1.z), leaf = __float_as_uint(q1.w);
-    float h0, h1;
-    bool hit = slab_one(lo, hi, r.ro, r.inv, r.tmin, boxes_finite && r.plain, &h0, &h1);
-    if (hit && leaf != 0) r.leaf = leaf;  // the miss link is where the walk goes on afterwards
-    r.node = (hit && leaf == 0) ? r.node + 1 : miss;
-}
-
-// The pending leaf of a lane: its primitives; the walk goes on at the miss link already in node.
-__device__ __forceinline__ void threaded_leaf(ThreadedRay& r, const PrimRec* __restrict__ prims, int32_t sphere_begin) {
-    const uint32_t beg = r.leaf & 0x0FFFFFFFu;
-    const uint32_t end = beg + ((r.leaf >> 28) & 7u) + 1u;
-    for (uint32_t s = beg; s < end; ++s) test_prim(prims, s, sphere_begin, r.ro, r.rd, &r.tmin, &r.u, &r.v, &r.prim);
-    r.leaf = 0;
-}
-
-
-// ---------------------------------------------------------------- stackless walk
-// One ray's walk over the walk records (rgpu_types.h: WalkNode). `node` is the link in hand: a
-// record's (>= 0 as a signed word), an entered leaf's primitive word (negative) or kInvalid once
-// the walk has ended. What is still to visit sits on a stack: the newest link in `tos`, the next
-// kWalkStackLds - 1 in the lane's column of the workgroup's LDS, deeper ones in private memory.
+// ---------------------------------------------------------------- the walk
+// One ray's walk over the walk records (rgpu_types.h: WalkNode), for every traversal variant.
+// `node` is the link in hand: a record's (>= 0 as a signed word), an entered leaf's primitive word
+// (negative) or kInvalid once the walk has ended. What is still to visit sits on a stack: the
+// newest link in `tos`, the next kWalkStackLds - 1 in the lane's column of the workgroup's LDS,
+// deeper ones in private memory.
 //
-// The walk enters the leaves that the reference's binary walk enters, in its order
-// (kernels/extension_ray_cast_stackless.cl:81-200), with the same far clip at each:
-//  - a record holds the four boxes two levels down, and a node's box is the union of its
+// The walk enters the leaves that the reference's walk of the variant enters, in its order, with
+// the same far clip at each. Stackless (kernels/extension_ray_cast_stackless.cl:81-200): the two
+// children of a node are tested together, the nearer goes first, the farther is deferred and
+// entered later without another test of its own box. Threaded (common/threaded_bvh.hpp:527-569,
+// 366-395): the children come in the order of the ray's direction class (or in the tree's own),
+// each tested with the far clip of its turn; the root is tested too.
+//  - A record holds the four boxes two levels down, and a node's box is the union of its
 //    children's. With finite, ordered boxes and a finite origin the slab products are monotone
 //    in the planes, rounding included, so the two children's entry and exit per axis are the
 //    minimum and maximum of the grandchildren's: one visit makes the decisions of a node and of
-//    the child that is entered next, and no leaf lies between them;
-//  - a child none of whose children is hit contributes nothing and is skipped;
-//  - the farther child is deferred as a half record and its two boxes are tested again when it
-//    is popped, with the far clip of that moment. Where one of them was hit and that one is a
+//    the child that is entered first, and no leaf lies between them;
+//  - a child none of whose children is hit contributes nothing and is skipped; what a far clip
+//    excludes, every smaller one does;
+//  - a child to visit later is deferred as a half record, whose two boxes are tested again when
+//    it is popped, with the far clip of that moment. Where one of them was hit and that one is a
 //    branch, its record is deferred directly: if the shrunk clip excludes its box, it excludes
-//    the boxes inside it.
+//    the boxes inside it. So does a grandchild that is a branch; one that is a leaf is deferred
+//    by its word (stackless) or as a single box to test again (threaded).
 // A wave with a ray or a scene that breaks the premise takes the binary visits one by one.
 //
-// Measured on 4.19 M incoherent rays over 1.3M triangles (persistent kernel): one 64-byte record
-// per binary node, leaves included, walked with a bitstack, a six-register short stack and parent
-// climbs took 1.12-1.16 ms: 25.1 dependent visits a ray, 8,478 VALU operations per 64 rays (84 %
-// busy at 38 % of the lanes) and 5.6 GB from beyond the L2. Links that need no decoding (a branch
-// link is the record's 16-byte index, a leaf link the primitive range itself) and a stack whose
-// push and pop are one LDS access: 1.00 ms. One 128-byte line for two levels, none for leaves:
-// 0.77 ms, 13.5 visits a ray, 5,800 VALU operations (76 % busy at 48 %), 3.4 GB (4.4 TB/s). Both
-// bounds are near; 8 waves per SIMD fetch more from beyond the L2 and are slower.
-struct StacklessRay {
+// Measured on 4.19 M incoherent rays over 1.3M triangles (persistent kernel). Stackless: one
+// 64-byte record per binary node, leaves included, walked with a bitstack, a six-register short
+// stack and parent climbs took 1.12-1.16 ms: 25.1 dependent visits a ray, 8,478 VALU operations
+// per 64 rays (84 % busy at 38 % of the lanes) and 5.6 GB from beyond the L2. Links that need no
+// decoding (a branch link is the record's 16-byte index, a leaf link the primitive range itself)
+// and a stack whose push and pop are one LDS access: 1.00 ms. One 128-byte line for two levels,
+// none for leaves: 0.77 ms, 13.5 visits a ray, 5,800 VALU operations (76 % busy at 48 %), 3.4 GB
+// (4.4 TB/s). Both bounds are near; 8 waves per SIMD fetch more from beyond the L2 and are
+// slower. Threaded: seven pre-ordered tables of 32-byte records (344 MB for that scene, 51.7 visits
+// a ray, 9.3 GB from beyond the L2 a launch) took 2.04 ms by direction class and 1.97 ms in the
+// tree's own order; the records that the stackless walk reads, with the child orders as bits, take
+// 0.90 and 1.09 ms, and the tables are gone from the scene (327,680 triangles: 57 -> 20 ms).
+struct WalkRay {
     F3 ro, rd, inv;
     float tmin, u, v;
     int32_t prim;
     bool plain, flat;  // the visits the ray allows (visit_kind, set once per ray)
+    uint32_t turn;     // threaded: first bit of the ray's direction class in an order word
     uint32_t node;
     uint32_t tos;   // newest deferred link; kInvalid when nothing is deferred
     int32_t sp;     // LDS byte of the stack's next free entry (past the end: in private memory)
@@ -305,7 +200,7 @@ struct WalkStack {
     __device__ __forceinline__ int32_t end() const { return base + 256 * (int32_t)kWalkStackLds; }
     __device__ __forceinline__ int32_t first() const { return base + 4 * (int32_t)(threadIdx.x & 63); }
     __device__ __forceinline__ uint32_t& entry(int32_t sp) const { return *reinterpret_cast<uint32_t*>(lds + sp); }
-    __device__ __forceinline__ void push(StacklessRay& r, uint32_t link) const {
+    __device__ __forceinline__ void push(WalkRay& r, uint32_t link) const {
         if (__builtin_expect(r.sp < end(), 1)) entry(r.sp) = r.tos;
         else spill[(uint32_t)(r.sp - end()) >> 8] = r.tos;
         r.sp += 256;
@@ -313,7 +208,7 @@ struct WalkStack {
     }
     // Into r.node; kInvalid from an empty stack (the entry below the first push holds it). The
     // LDS read is unconditional, so that it stays an LDS read.
-    __device__ __forceinline__ void pop(StacklessRay& r) const {
+    __device__ __forceinline__ void pop(WalkRay& r) const {
         r.node = r.tos;
         r.sp = max(r.sp - 256, base);
         r.tos = entry(min(r.sp, end() - 4));
@@ -325,29 +220,16 @@ struct WalkStack {
 __device__ __forceinline__ int32_t wave_scalar(int32_t x) { return __builtin_amdgcn_readfirstlane(x); }
 
 // The kernel's dynamic LDS: `top` walk records (the top levels of the tree, numbered breadth-first
-// by the scene packer) without their padding, then kWalkStackLds words per lane, wave by wave.
-// Seven 16-byte words a record: an odd stride spreads the lanes' records over the banks.
+// by the scene packer) without their last 16 bytes, then (kVariantThreaded) their order words, then
+// kWalkStackLds words per lane, wave by wave. Seven 16-byte words a record: an odd stride spreads
+// the lanes' records over the banks.
 extern __shared__ float4 walk_lds[];
 
+template <int kVariant>
 __device__ __forceinline__ WalkStack walk_stack(uint32_t top, uint32_t* spill) {
     const uint32_t wave = (uint32_t)wave_scalar((int32_t)(threadIdx.x >> 6));
     return WalkStack{reinterpret_cast<char*>(walk_lds), spill,
-                     (int32_t)(kStagedBytes * top + wave * (256u * kWalkStackLds))};
-}
-
-__device__ __forceinline__ void stackless_begin(StacklessRay& r, const WalkStack& stk, uint32_t root, F3 ro, F3 rd,
-                                                float tmax) {
-    r.ro = ro;
-    r.rd = rd;
-    r.inv = f3(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
-    r.plain = plain_slabs(true, ro, r.inv) && tmax >= 0.0f;
-    r.flat = flat_slabs(ro, r.inv) && tmax >= 0.0f;
-    r.tmin = tmax;
-    r.u = r.v = 0.0f;
-    r.prim = -1;
-    r.node = root;
-    r.tos = kInvalid;
-    r.sp = stk.first();
+                     (int32_t)(staged_bytes(kVariant, top) + wave * (256u * kWalkStackLds))};
 }
 
 // How the rays of a wave may visit records (a scalar): kVisitPlain when no slab product can be
@@ -356,7 +238,7 @@ __device__ __forceinline__ void stackless_begin(StacklessRay& r, const WalkStack
 // otherwise kVisitBinary. A primitive test may accept a t that is NaN (of overflowed products):
 // no box passes that clip, which only the binary visit's comparisons tell.
 enum { kVisitBinary = 0, kVisitFlat = 1, kVisitPlain = 2 };
-__device__ __forceinline__ int32_t visit_kind(const StacklessRay& r, bool boxes_finite) {
+__device__ __forceinline__ int32_t visit_kind(const WalkRay& r, bool boxes_finite) {
     const bool dead = r.node == kInvalid, ok = boxes_finite && r.tmin == r.tmin;
     const int32_t kind = __all(dead || (ok && r.plain))                ? kVisitPlain
                          : __all(dead || (ok && (r.plain || r.flat))) ? kVisitFlat
@@ -364,13 +246,18 @@ __device__ __forceinline__ int32_t visit_kind(const StacklessRay& r, bool boxes_
     return wave_scalar(kind);
 }
 // The same after primitive tests, which only change clips.
-__device__ __forceinline__ int32_t visit_kind_after(int32_t kind, const StacklessRay& r) {
+__device__ __forceinline__ int32_t visit_kind_after(int32_t kind, const WalkRay& r) {
     return __all(r.tmin == r.tmin) ? kind : (int32_t)kVisitBinary;
 }
 
 // Stages the first `top` records at the start of walk_lds (the whole workgroup; barrier after).
+template <int kVariant>
 __device__ __forceinline__ void stage_records(const float4* __restrict__ recs, uint32_t top) {
     for (uint32_t j = threadIdx.x; j < 7u * top; j += blockDim.x) walk_lds[j] = recs[8u * (j / 7u) + j % 7u];
+    if constexpr (kVariant == kVariantThreaded) {
+        uint32_t* order = reinterpret_cast<uint32_t*>(walk_lds + 7u * top);
+        for (uint32_t j = threadIdx.x; j < top; j += blockDim.x) order[j] = __float_as_uint(recs[8u * j + 7u].x);
+    }
     __syncthreads();
 }
 
@@ -453,19 +340,23 @@ __device__ __forceinline__ BoxPlanes join(const BoxPlanes& a, const BoxPlanes& b
 struct WalkRecord {
     BoxPlanes box[4];
     WalkLinks link;
+    uint32_t order;  // kVariantThreaded
 };
 // kTop: records below link `top8` (8 * records) come from LDS.
-template <bool kTop>
+template <bool kTop, int kVariant>
 __device__ __forceinline__ void load_record(uint32_t at, const float4* __restrict__ recs, uint32_t top8, WalkRecord* r) {
     WalkWords q[6];
     if (kTop && at < top8) {
         const auto* p = (const LdsSpace WalkWords*)((const LdsSpace char*)walk_lds + __umul24(at, kStagedBytes / 8u));
         for (int k = 0; k < 6; ++k) q[k] = p[k];
         r->link = *(const LdsSpace WalkLinks*)(p + 6);
+        if constexpr (kVariant == kVariantThreaded)
+            r->order = *(const LdsSpace uint32_t*)((const LdsSpace char*)walk_lds + __umul24(top8, kStagedBytes / 8u) + at / 2u);
     } else {
         const auto* p = (const GlobalSpace WalkWords*)recs + at;
         for (int k = 0; k < 6; ++k) q[k] = p[k];
         r->link = *(const GlobalSpace WalkLinks*)(p + 6);
+        if constexpr (kVariant == kVariantThreaded) r->order = *(const GlobalSpace uint32_t*)(p + 7);
     }
     for (int h = 0; h < 2; ++h) {
         const WalkWords a = q[3 * h], b = q[3 * h + 1], c = q[3 * h + 2];
@@ -476,36 +367,54 @@ __device__ __forceinline__ void load_record(uint32_t at, const float4* __restric
 
 // Visit of the record `node` names: descent two levels down, what else is hit deferred, or a pop
 // when nothing is hit. kKind: kVisitPlain or kVisitFlat.
-template <bool kTop, int kKind>
-__device__ __forceinline__ void stackless_visit(StacklessRay& r, const WalkStack& stk, const float4* __restrict__ recs,
-                                                uint32_t top8) {
+template <int kVariant, bool kTop, int kKind>
+__device__ __forceinline__ void walk_visit(WalkRay& r, const WalkStack& stk, const float4* __restrict__ recs,
+                                           uint32_t top8) {
+    constexpr bool kNear = kVariant == kVariantStackless;  // else in the order of the tables
     uint32_t at = r.node & ~7u;
-    const uint32_t only = r.node & 7u;  // kFirstHalf, kSecondHalf or 0
+    const uint32_t only = r.node & 7u;  // kFirstHalf, kSecondHalf, kOneBox + k or 0
     // (an opaque, different start keeps the compiler from joining the two kinds' common part,
     // which would hold all 24 products of a record in registers)
     if (kKind == kVisitPlain) asm("; plain visit" : "+v"(at));
     else asm("; flat visit" : "+v"(at));
     WalkRecord w;
-    load_record<kTop>(at, recs, top8, &w);
+    load_record<kTop, kVariant>(at, recs, top8, &w);
     const BoxSlabs s0 = box_slabs<kKind>(w.box[0], r.ro, r.inv), s1 = box_slabs<kKind>(w.box[1], r.ro, r.inv);
-    const Span c0 = clipped(s0.clip(), r.tmin), c1 = clipped(s1.clip(), r.tmin);
+    Span c0 = clipped(s0.clip(), r.tmin), c1 = clipped(s1.clip(), r.tmin);
     const Span L = clipped(join(s0, s1).clip(), r.tmin);
     const BoxSlabs s2 = box_slabs<kKind>(w.box[2], r.ro, r.inv), s3 = box_slabs<kKind>(w.box[3], r.ro, r.inv);
-    const Span c2 = clipped(s2.clip(), r.tmin), c3 = clipped(s3.clip(), r.tmin);
+    Span c2 = clipped(s2.clip(), r.tmin), c3 = clipped(s3.clip(), r.tmin);
     const Span R = clipped(join(s2, s3).clip(), r.tmin);
+    // what the link leaves out is not hit
+    bool half0 = only != kSecondHalf, half1 = only != kFirstHalf;
+    bool firstL, turnL = false, turnR = false;
+    if constexpr (kNear) {
+        firstL = nearer(L, R);
+    } else {
+        const uint32_t mask = 0x84210C3Fu >> (4u * only);
+        const float none = __builtin_inff();
+        c0.enter = (mask & 1u) ? c0.enter : none;
+        c1.enter = (mask & 2u) ? c1.enter : none;
+        c2.enter = (mask & 4u) ? c2.enter : none;
+        c3.enter = (mask & 8u) ? c3.enter : none;
+        half0 = half1 = true;
+        const uint32_t turns = kVariant == kVariantThreaded ? w.order >> r.turn : 0u;
+        firstL = (turns & 1u) == 0;
+        turnL = (turns & 2u) != 0;
+        turnR = (turns & 4u) != 0;
+    }
     // (a leaf child's second box is its first again, so it changes neither union nor these)
-    const bool aliveL = (c0.hit() || c1.hit()) && only != kSecondHalf;
-    const bool aliveR = (c2.hit() || c3.hit()) && only != kFirstHalf;
-    const bool takeL = aliveL && (nearer(L, R) || !aliveR);
+    const bool aliveL = (c0.hit() || c1.hit()) && half0, aliveR = (c2.hit() || c3.hit()) && half1;
+    const bool takeL = aliveL && (firstL || !aliveR);
     if (aliveL && aliveR) {
-        // the other half: as a half of this record; directly where that is exact (a leaf child of
-        // the node itself, whose second link is empty, or a single branch child hit)
+        // the other half: as a half of this record; directly where that is exact (a single branch
+        // child hit; stackless, a leaf child of the node itself, whose second link is empty)
         const uint32_t oa = takeL ? w.link.z : w.link.x, ob = takeL ? w.link.w : w.link.y;
         const Span ga{takeL ? c2.enter : c0.enter, takeL ? c2.leave : c0.leave};
         const Span gb{takeL ? c3.enter : c1.enter, takeL ? c3.leave : c1.leave};
         const uint32_t one = ga.hit() ? oa : ob;
         const bool both = ga.hit() && gb.hit();
-        const bool direct = ob == kInvalid || (!both && (int32_t)one >= 0);
+        const bool direct = (kNear && ob == kInvalid) || (!both && (int32_t)one >= 0);
         stk.push(r, direct ? one : (at | (takeL ? kSecondHalf : kFirstHalf)));
     }
     if (aliveL || aliveR) {
@@ -514,23 +423,47 @@ __device__ __forceinline__ void stackless_visit(StacklessRay& r, const WalkStack
         const Span b{takeL ? c1.enter : c3.enter, takeL ? c1.leave : c3.leave};
         const uint32_t la = takeL ? w.link.x : w.link.z, lb = takeL ? w.link.y : w.link.w;
         const bool ha = a.hit(), hb = b.hit() && lb != kInvalid;
-        const bool takeA = ha && (nearer(a, b) || !hb);
+        bool firstA;
+        if constexpr (kNear) firstA = nearer(a, b);
+        else firstA = takeL ? !turnL : !turnR;
+        const bool takeA = ha && (firstA || !hb);
         r.node = takeA ? la : lb;
-        if (ha && hb) stk.push(r, takeA ? lb : la);
+        if (ha && hb) {
+            uint32_t later = takeA ? lb : la;
+            if (!kNear && (int32_t)later < 0) later = at | (kOneBox + (takeL ? 0u : 2u) + (takeA ? 1u : 0u));
+            stk.push(r, later);
+        }
     } else {
         stk.pop(r);
     }
 }
 
-// The same walk one binary node at a time, as the reference visits them: a record's node itself
-// first (its two children, boxed by the unions of the records' boxes), then each entered half.
-// For waves that no other kind fits, and for the event counts.
+__device__ __forceinline__ float pick(float a, float b, float c, float d, uint32_t k) {
+    const float l = (k & 1u) ? b : a, h = (k & 1u) ? d : c;
+    return (k & 2u) ? h : l;
+}
+__device__ __forceinline__ BoxPlanes pick_box(const WalkRecord& w, uint32_t k) {
+    const BoxPlanes a = w.box[0], b = w.box[1], c = w.box[2], d = w.box[3];
+    return BoxPlanes{{pick(a.lo[0], b.lo[0], c.lo[0], d.lo[0], k), pick(a.lo[1], b.lo[1], c.lo[1], d.lo[1], k),
+                      pick(a.lo[2], b.lo[2], c.lo[2], d.lo[2], k)},
+                     {pick(a.hi[0], b.hi[0], c.hi[0], d.hi[0], k), pick(a.hi[1], b.hi[1], c.hi[1], d.hi[1], k),
+                      pick(a.hi[2], b.hi[2], c.hi[2], d.hi[2], k)}};
+}
+__device__ __forceinline__ uint32_t pick_link(const WalkRecord& w, uint32_t k) {
+    const uint32_t l = (k & 1u) ? w.link.y : w.link.x, h = (k & 1u) ? w.link.w : w.link.z;
+    return (k & 2u) ? h : l;
+}
+
+// The same walk one binary node at a time, as the reference visits them. For waves that no other
+// kind fits, and for the event counts.
+// Stackless: a record's node itself first (its two children, boxed by the unions of the record's
+// boxes), then each entered half.
 template <bool kTop, bool kCount>
-__device__ __forceinline__ void stackless_visit_binary(StacklessRay& r, const WalkStack& stk,
+__device__ __forceinline__ void stackless_visit_binary(WalkRay& r, const WalkStack& stk,
                                                        const float4* __restrict__ recs, uint32_t top8, Cnt* cnt) {
     const uint32_t at = r.node & ~7u, only = r.node & 7u;
     WalkRecord w;
-    load_record<kTop>(at, recs, top8, &w);
+    load_record<kTop, kVariantStackless>(at, recs, top8, &w);
     BoxPlanes A, B;
     uint32_t la, lb;
     if (only == 0) {
@@ -540,11 +473,11 @@ __device__ __forceinline__ void stackless_visit_binary(StacklessRay& r, const Wa
         la = w.link.y == kInvalid ? w.link.x : at | kFirstHalf;
         lb = w.link.w == kInvalid ? w.link.z : at | kSecondHalf;
     } else {
-        const bool first = only == kFirstHalf;
-        A = first ? w.box[0] : w.box[2];
-        B = first ? w.box[1] : w.box[3];
-        la = first ? w.link.x : w.link.z;
-        lb = first ? w.link.y : w.link.w;
+        const uint32_t k = only == kFirstHalf ? 0u : 2u;
+        A = pick_box(w, k);
+        B = pick_box(w, k + 1u);
+        la = pick_link(w, k);
+        lb = pick_link(w, k + 1u);
     }
     const Slab a = box_slabs<kVisitBinary>(A, r.ro, r.inv).clip(), b = box_slabs<kVisitBinary>(B, r.ro, r.inv).clip();
     const bool ha = a.hit(r.tmin), hb = b.hit(r.tmin);
@@ -557,23 +490,90 @@ __device__ __forceinline__ void stackless_visit_binary(StacklessRay& r, const Wa
     if (ha && hb) stk.push(r, takeA ? lb : la);
     if (!(ha || hb)) stk.pop(r);
 }
+// Threaded: every node is tested once, in its turn. A record's node (its box passed): the child
+// whose turn is first, then its children while it is hit; the other child is deferred as its half,
+// a second grandchild as its box.
+template <int kVariant, bool kTop, bool kCount>
+__device__ __forceinline__ void threaded_visit_binary(WalkRay& r, const WalkStack& stk,
+                                                      const float4* __restrict__ recs, uint32_t top8, Cnt* cnt) {
+    const uint32_t at = r.node & ~7u, only = r.node & 7u;
+    WalkRecord w;
+    load_record<kTop, kVariant>(at, recs, top8, &w);
+    const uint32_t turns = kVariant == kVariantThreaded ? w.order >> r.turn : 0u;
+    auto test = [&](const BoxPlanes& b) {
+        if (kCount) cnt->node++;
+        return box_slabs<kVisitBinary>(b, r.ro, r.inv).clip().hit(r.tmin);
+    };
+    uint32_t k = only & 3u;  // the box to test last
+    bool passed;             // whether the half that holds it is entered
+    if (only >= kOneBox) {
+        passed = true;
+    } else {
+        uint32_t half = only == 0 ? turns & 1u : only - kFirstHalf;
+        passed = test(join(pick_box(w, 2u * half), pick_box(w, 2u * half + 1u)));
+        if (only == 0 && passed) {
+            stk.push(r, at | (half != 0 ? kFirstHalf : kSecondHalf));
+        } else if (only == 0) {
+            half ^= 1u;
+            passed = test(join(pick_box(w, 2u * half), pick_box(w, 2u * half + 1u)));
+        }
+        if (passed && pick_link(w, 2u * half + 1u) == kInvalid) {  // a leaf child: entered by its word
+            r.node = pick_link(w, 2u * half);
+            return;
+        }
+        k = 2u * half + ((turns >> (1u + half)) & 1u);
+        if (passed && test(pick_box(w, k))) {
+            stk.push(r, at | (kOneBox + (k ^ 1u)));
+            r.node = pick_link(w, k);
+            return;
+        }
+        k ^= 1u;
+    }
+    if (passed && test(pick_box(w, k))) r.node = pick_link(w, k);
+    else stk.pop(r);
+}
 
-template <bool kTop, bool kCount>
-__device__ __forceinline__ void stackless_visit_as(int32_t kind, StacklessRay& r, const WalkStack& stk,
-                                                   const float4* __restrict__ recs, uint32_t top, Cnt* cnt) {
-    if (!kCount && kind == kVisitPlain) stackless_visit<kTop, kVisitPlain>(r, stk, recs, 8 * top);
-    else if (!kCount && kind == kVisitFlat) stackless_visit<kTop, kVisitFlat>(r, stk, recs, 8 * top);
-    else stackless_visit_binary<kTop, kCount>(r, stk, recs, 8 * top, cnt);
+template <int kVariant, bool kTop, bool kCount>
+__device__ __forceinline__ void walk_visit_as(int32_t kind, WalkRay& r, const WalkStack& stk,
+                                              const float4* __restrict__ recs, uint32_t top, Cnt* cnt) {
+    if (!kCount && kind == kVisitPlain) walk_visit<kVariant, kTop, kVisitPlain>(r, stk, recs, 8 * top);
+    else if (!kCount && kind == kVisitFlat) walk_visit<kVariant, kTop, kVisitFlat>(r, stk, recs, 8 * top);
+    else if constexpr (kVariant == kVariantStackless)
+        stackless_visit_binary<kTop, kCount>(r, stk, recs, 8 * top, cnt);
+    else
+        threaded_visit_binary<kVariant, kTop, kCount>(r, stk, recs, 8 * top, cnt);
+}
+
+template <int kVariant, bool kCount>
+__device__ __forceinline__ void walk_begin(WalkRay& r, const WalkStack& stk, const TraceScene& sc, F3 ro, F3 rd,
+                                           float tmax, Cnt* cnt) {
+    r.ro = ro;
+    r.rd = rd;
+    r.inv = f3(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
+    r.plain = plain_slabs(true, ro, r.inv) && tmax >= 0.0f;
+    r.flat = flat_slabs(ro, r.inv) && tmax >= 0.0f;
+    r.tmin = tmax;
+    r.u = r.v = 0.0f;
+    r.prim = -1;
+    r.node = sc.root;
+    r.tos = kInvalid;
+    r.sp = stk.first();
+    if constexpr (kVariant != kVariantStackless) {
+        r.turn = 3u * direction_class(rd);
+        const BoxPlanes root{{sc.root_lo[0], sc.root_lo[1], sc.root_lo[2]}, {sc.root_hi[0], sc.root_hi[1], sc.root_hi[2]}};
+        if (!box_slabs<kVisitBinary>(root, ro, r.inv).clip().hit(tmax)) r.node = kInvalid;
+        if (kCount) cnt->node++;
+    }
 }
 
 // The primitives of an entered leaf, then the pop.
-template <bool kCount>
-__device__ __forceinline__ void stackless_leaf(StacklessRay& r, const WalkStack& stk,
-                                               const PrimRec* __restrict__ prims, int32_t sphere_begin, Cnt* cnt) {
+template <int kVariant, bool kCount>
+__device__ __forceinline__ void walk_leaf(WalkRay& r, const WalkStack& stk, const PrimRec* __restrict__ prims,
+                                          int32_t sphere_begin, Cnt* cnt) {
     const uint32_t beg = r.node & 0x0FFFFFFFu;
     const uint32_t end = beg + ((r.node >> 28) & 7u) + 1u;
     if (kCount) {
-        cnt->leaf++;
+        cnt->leaf += kVariant == kVariantStackless ? 1u : 0u;
         cnt->prim += end - beg;
     }
     for (uint32_t s = beg; s < end; ++s) test_prim(prims, s, sphere_begin, r.ro, r.rd, &r.tmin, &r.u, &r.v, &r.prim);
@@ -581,14 +581,11 @@ __device__ __forceinline__ void stackless_leaf(StacklessRay& r, const WalkStack&
     if (kCount) cnt->step(false, false);
 }
 
-// Lane states of the resumable walks: live (a ray in progress), pending (stopped at an entered
-// leaf whose primitives are not yet tested), walking (at a record to visit).
-__device__ __forceinline__ bool walk_live(const StacklessRay& r) { return r.node != kInvalid; }
-__device__ __forceinline__ bool walk_pending(const StacklessRay& r) { return (int32_t)r.node < -1; }
-__device__ __forceinline__ bool walk_walking(const StacklessRay& r) { return (int32_t)r.node >= 0; }
-__device__ __forceinline__ bool walk_live(const ThreadedRay& r) { return r.node != kInvalid || r.leaf != 0; }
-__device__ __forceinline__ bool walk_pending(const ThreadedRay& r) { return r.leaf != 0; }
-__device__ __forceinline__ bool walk_walking(const ThreadedRay& r) { return r.node != kInvalid && r.leaf == 0; }
+// Lane states: live (a ray in progress), pending (stopped at an entered leaf whose primitives are
+// not yet tested), walking (at a record to visit).
+__device__ __forceinline__ bool walk_live(const WalkRay& r) { return r.node != kInvalid; }
+__device__ __forceinline__ bool walk_pending(const WalkRay& r) { return (int32_t)r.node < -1; }
+__device__ __forceinline__ bool walk_walking(const WalkRay& r) { return (int32_t)r.node >= 0; }
 
 __device__ __forceinline__ uint32_t count_lanes(bool b) { return (uint32_t)__popcll(__ballot(b)); }
 
@@ -601,47 +598,26 @@ template <int kVariant, bool kTop = false, bool kCount = false>
 __device__ __forceinline__ int32_t trace_batched(const TraceScene& sc, F3 ro, F3 rd, float* tmin_io, float* uo,
                                                  float* vo, uint32_t leaf_batch, uint32_t top = 0,
                                                  Cnt* cnt = nullptr) {
-    if constexpr (kVariant == kVariantStackless) {
-        uint32_t spill[kWalkStackSpill];
-        const WalkStack stk = walk_stack(top, spill);
-        const float4* recs = reinterpret_cast<const float4*>(sc.walk_nodes);
-        StacklessRay st;
-        stackless_begin(st, stk, sc.root, ro, rd, *tmin_io);
-        int32_t kind = visit_kind(st, sc.boxes_finite != 0);
-        for (;;) {
-            const uint32_t nwalk = count_lanes(walk_walking(st)), npending = count_lanes(walk_pending(st));
-            if (nwalk + npending == 0) break;
-            if (npending >= leaf_batch || npending >= nwalk) {
-                if (walk_pending(st)) stackless_leaf<kCount>(st, stk, sc.prims, sc.sphere_begin, cnt);
-                kind = visit_kind_after(kind, st);
-            } else if (walk_walking(st)) {
-                stackless_visit_as<kTop, kCount>(kind, st, stk, recs, top, cnt);
-            }
+    uint32_t spill[kWalkStackSpill];
+    const WalkStack stk = walk_stack<kVariant>(top, spill);
+    const float4* recs = reinterpret_cast<const float4*>(sc.walk_nodes);
+    WalkRay st;
+    walk_begin<kVariant, kCount>(st, stk, sc, ro, rd, *tmin_io, cnt);
+    int32_t kind = visit_kind(st, sc.boxes_finite != 0);
+    for (;;) {
+        const uint32_t nwalk = count_lanes(walk_walking(st)), npending = count_lanes(walk_pending(st));
+        if (nwalk + npending == 0) break;
+        if (npending >= leaf_batch || npending >= nwalk) {
+            if (walk_pending(st)) walk_leaf<kVariant, kCount>(st, stk, sc.prims, sc.sphere_begin, cnt);
+            kind = visit_kind_after(kind, st);
+        } else if (walk_walking(st)) {
+            walk_visit_as<kVariant, kTop, kCount>(kind, st, stk, recs, top, cnt);
         }
-        *tmin_io = st.tmin;
-        *uo = st.u;
-        *vo = st.v;
-        return st.prim;
-    } else {
-        ThreadedRay st;
-        threaded_begin<kVariant>(st, sc.mt_nodes, sc.nnodes, ro, rd, *tmin_io);
-        const bool finite = sc.boxes_finite != 0;
-        for (;;) {
-            if (__ballot(walk_live(st)) == 0) break;
-            const bool pending = walk_pending(st);
-            const bool walking = walk_walking(st);
-            const uint32_t npending = count_lanes(pending);
-            if (npending >= leaf_batch || npending >= count_lanes(walking)) {
-                if (pending) threaded_leaf(st, sc.prims, sc.sphere_begin);
-            } else if (walking) {
-                threaded_visit(st, finite);
-            }
-        }
-        *tmin_io = st.tmin;
-        *uo = st.u;
-        *vo = st.v;
-        return st.prim;
     }
+    *tmin_io = st.tmin;
+    *uo = st.u;
+    *vo = st.v;
+    return st.prim;
 }
 
 }  // namespace rgpu

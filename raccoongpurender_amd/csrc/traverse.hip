@@ -1,5 +1,5 @@
-// Extension ray casting on gfx950: stackless (parent-pointer) and threaded
-// (skip-pointer, six direction tables) BVH2 traversal.
+// Extension ray casting on gfx950: the stackless (parent-pointer) and threaded (skip-pointer, six
+// direction orders or the tree's own) BVH2 traversals.
 //
 // Reference behaviour (kernels/extension_ray_cast_stackless.cl:81-246,
 // kernels/extension_ray_cast.cl:44-94, kernels/slab.cl, kernels/intersect_triangle.cl):
@@ -11,13 +11,10 @@
 // library is built with -ffp-contract=off, so hit index, t, u and v are bit-identical
 // to the oracle on the same tree.
 //
-// Layout (rgpu_types.h): stackless walk records are 128 B, one per two tree levels (a leaf needs
-// none), threaded records are 32 B in one pre-ordered table per ray direction class, primitives
-// are 48 B records in leaf order.
+// Layout (rgpu_types.h): walk records are 128 B, one per two tree levels (a leaf needs none);
+// primitives are 48 B records in leaf order.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-
-#include <type_traits>
 
 #include "rgpu_traverse.h"
 #include "rgpu_types.h"
@@ -57,16 +54,11 @@ __device__ __forceinline__ void flush_counts(unsigned long long* counters, const
     wave_add(counters + 4, c.node);
 }
 
-// One thread per ray, in three forms of the same walk (same visits, same results): plain, the
-// walk as one loop; count, the same with event counters; batched, leaves batched across the wave
-// (chosen by a leaf_batch above 1). The stackless walk's plain and counting forms are its batched
-// loop with leaf_batch 1.
-enum { kWalkPlain = 0, kWalkCount = 1, kWalkBatched = 2 };
-
-template <bool kCount>
-__global__ void __launch_bounds__(256, 8) k_trace_stackless(const TraceRay* __restrict__ rays,
-                                                         TraceHit* __restrict__ hits, uint32_t n, TraceScene sc,
-                                                         uint32_t leaf_batch, unsigned long long* counters) {
+// One thread per ray; kCount: with event counters (and the binary visits that they count).
+template <int kVariant, bool kCount>
+__global__ void __launch_bounds__(256, 8) k_trace_rays(const TraceRay* __restrict__ rays, TraceHit* __restrict__ hits,
+                                                       uint32_t n, TraceScene sc, uint32_t leaf_batch,
+                                                       unsigned long long* counters) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     Cnt c;
     if (i < n) {
@@ -74,33 +66,10 @@ __global__ void __launch_bounds__(256, 8) k_trace_stackless(const TraceRay* __re
         float t;
         load_ray(rays, i, &ro, &rd, &t);
         float u, v;
-        const int32_t prim =
-            trace_batched<kVariantStackless, false, kCount>(sc, ro, rd, &t, &u, &v, leaf_batch, 0, &c);
+        const int32_t prim = trace_batched<kVariant, false, kCount>(sc, ro, rd, &t, &u, &v, leaf_batch, 0, &c);
         store_hit(hits, i, prim, t, u, v);
     }
     if (kCount) flush_counts(counters, c);
-}
-
-// kVariant: kVariantThreaded (a table per direction class) or kVariantSingleThreaded.
-template <int kMode, int kVariant>
-__global__ void __launch_bounds__(256) k_trace_threaded(const TraceRay* __restrict__ rays,
-                                                        TraceHit* __restrict__ hits, uint32_t n, TraceScene sc,
-                                                        uint32_t leaf_batch, unsigned long long* counters) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    Cnt c;
-    if (i < n) {
-        F3 ro, rd;
-        float t;
-        load_ray(rays, i, &ro, &rd, &t);
-        float u, v;
-        int32_t prim = kMode == kWalkBatched
-                           ? trace_batched<kVariant>(sc, ro, rd, &t, &u, &v, leaf_batch)
-                           : trace_threaded<kMode == kWalkCount, kVariant>(sc.mt_nodes, sc.nnodes, sc.prims,
-                                                                           sc.sphere_begin, sc.boxes_finite != 0, ro,
-                                                                           rd, &t, &u, &v, &c);
-        store_hit(hits, i, prim, t, u, v);
-    }
-    if (kMode == kWalkCount) flush_counts(counters, c);
 }
 
 // Persistent wave64 traversal: wave w owns rays [w * chunk, (w + 1) * chunk) and hands them to
@@ -112,18 +81,17 @@ __global__ void __launch_bounds__(256) k_trace_threaded(const TraceRay* __restri
 // once `leaf_batch` lanes wait at leaves or at least as many lanes wait as walk on, so that the
 // primitive tests run with many lanes at once instead of taxing every node visit of the wave. Each ray still
 // visits its nodes and tests its primitives in the order of the one-ray walk.
-// Stackless: the first `top` walk records (the top of the tree, numbered breadth-first) are
-// copied to LDS at the start and read from there (walk_lds: the records, then the stacks).
+// The first `top` walk records (the top of the tree, numbered breadth-first) are copied to LDS at
+// the start and read from there (walk_lds).
 template <int kVariant>
-__global__ void __launch_bounds__(256, kVariant == kVariantStackless ? 7 : 1) k_trace_persistent(const TraceRay* __restrict__ rays,
+__global__ void __launch_bounds__(256, 7) k_trace_persistent(const TraceRay* __restrict__ rays,
                                                           TraceHit* __restrict__ hits, uint32_t n, TraceScene sc,
                                                           uint32_t chunk, uint32_t refill, uint32_t leaf_batch,
                                                           uint32_t top) {
-    constexpr bool kStackless = kVariant == kVariantStackless;
-    uint32_t spill[kStackless ? kWalkStackSpill : 1];
-    const WalkStack stk = walk_stack(top, spill);
+    uint32_t spill[kWalkStackSpill];
+    const WalkStack stk = walk_stack<kVariant>(top, spill);
     const float4* recs = reinterpret_cast<const float4*>(sc.walk_nodes);
-    if constexpr (kStackless) stage_records(recs, top);
+    stage_records<kVariant>(recs, top);
     const uint32_t lane = threadIdx.x & 63;
     // the wave's cursor in scalar registers, so that the loop's control costs no vector operations
     const uint32_t wave = (uint32_t)wave_scalar((int32_t)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
@@ -131,10 +99,8 @@ __global__ void __launch_bounds__(256, kVariant == kVariantStackless ? 7 : 1) k_
     uint64_t next = (uint64_t)wave * chunk;
     const uint64_t end = next + chunk < (uint64_t)n ? next + chunk : (uint64_t)n;
     uint32_t ray = kInvalid;
-    using State = typename std::conditional<kStackless, StacklessRay, ThreadedRay>::type;
-    State st;
+    WalkRay st;
     st.node = kInvalid;
-    if constexpr (!kStackless) st.leaf = 0;
     const bool finite = sc.boxes_finite != 0;
     int32_t kind = 0;  // a scalar: how the live rays may visit records
     for (;;) {
@@ -152,28 +118,20 @@ __global__ void __launch_bounds__(256, kVariant == kVariantStackless ? 7 : 1) k_
                     F3 ro, rd;
                     float tmax;
                     load_ray(rays, ray, &ro, &rd, &tmax);
-                    if constexpr (kStackless) stackless_begin(st, stk, sc.root, ro, rd, tmax);
-                    else threaded_begin<kVariant>(st, sc.mt_nodes, sc.nnodes, ro, rd, tmax);
+                    walk_begin<kVariant, false>(st, stk, sc, ro, rd, tmax, nullptr);
                 }
             }
             if (next >= end) break;  // every lane was idle and nothing is left to hand out
             next += nidle;
-            if constexpr (kStackless) kind = visit_kind(st, finite);
+            kind = visit_kind(st, finite);
             nwalk = count_lanes(walk_walking(st));
             npending = count_lanes(walk_pending(st));
         }
         if (npending >= leaf_batch || npending >= nwalk) {
-            if (walk_pending(st)) {
-                if constexpr (kStackless) stackless_leaf<false>(st, stk, sc.prims, sc.sphere_begin, nullptr);
-                else threaded_leaf(st, sc.prims, sc.sphere_begin);
-            }
-            if constexpr (kStackless) kind = visit_kind_after(kind, st);
+            if (walk_pending(st)) walk_leaf<kVariant, false>(st, stk, sc.prims, sc.sphere_begin, nullptr);
+            kind = visit_kind_after(kind, st);
         } else if (walk_walking(st)) {
-            if constexpr (kStackless) {
-                stackless_visit_as<true, false>(kind, st, stk, recs, top, nullptr);
-            } else {
-                threaded_visit(st, finite);
-            }
+            walk_visit_as<kVariant, true, false>(kind, st, stk, recs, top, nullptr);
         }
     }
 }
@@ -190,78 +148,54 @@ __global__ void __launch_bounds__(256) k_trace_empty(const TraceRay* __restrict_
 }
 
 template <int kVariant>
-void launch_threaded(int mode, dim3 grid, uint32_t block, hipStream_t stream, const TraceRay* rays, TraceHit* hits,
-                     uint32_t n, const TraceScene& sc, uint32_t leaf_batch, unsigned long long* counters) {
-    if (mode == kWalkCount)
-        hipLaunchKernelGGL((k_trace_threaded<kWalkCount, kVariant>), grid, dim3(block), 0, stream, rays, hits, n, sc,
-                           leaf_batch, counters);
-    else if (mode == kWalkBatched)
-        hipLaunchKernelGGL((k_trace_threaded<kWalkBatched, kVariant>), grid, dim3(block), 0, stream, rays, hits, n, sc,
-                           leaf_batch, counters);
+hipError_t launch_variant(const TraceScene& sc, const TraceRay* rays, TraceHit* hits, uint32_t n, uint32_t block,
+                          hipStream_t stream, unsigned long long* counters, const TraceTuning& tune) {
+    if (block == 0 && !counters) {
+        // persistent kernel: as many resident waves as the launch asks for, each with a chunk of
+        // the rays
+        const uint32_t cus = tune.cu_count ? tune.cu_count : 256u;
+        const uint32_t wps = tune.waves_per_simd ? tune.waves_per_simd : kDefaultWaves;
+        const uint32_t refill = tune.refill ? tune.refill : kDefaultRefill;
+        const uint32_t leaf_batch = tune.leaf_batch ? tune.leaf_batch : kDefaultLeafBatch;
+        const uint32_t blocks = cus * wps;  // 4 waves (one per SIMD) per 256-thread block
+        const uint32_t waves = blocks * 4u;
+        const uint32_t chunk = (n + waves - 1) / waves;
+        uint32_t top = tune.treelet ? tune.treelet : kDefaultTreelet;
+        if (top == kTreeletOff) top = 0;
+        top = top < sc.nwalk ? top : sc.nwalk;
+        top = top < kTreeletMaxStaged ? top : kTreeletMaxStaged;
+        hipLaunchKernelGGL(k_trace_persistent<kVariant>, dim3(blocks), dim3(256), walk_lds_bytes(kVariant, top, 256),
+                           stream, rays, hits, n, sc, chunk, refill, leaf_batch, top);
+        return hipGetLastError();
+    }
+    if (block == 0) block = 256;
+    const dim3 grid((n + block - 1) / block);
+    const size_t lds = walk_lds_bytes(kVariant, 0, block);
+    // leaves batched by default only once as many lanes wait at leaves as walk on (64; 1: every
+    // lane's leaf at once)
+    const uint32_t leaf_batch = tune.leaf_batch ? tune.leaf_batch : kPerRayLeafBatch;
+    if (counters)
+        hipLaunchKernelGGL((k_trace_rays<kVariant, true>), grid, dim3(block), lds, stream, rays, hits, n, sc, 1u,
+                           counters);
     else
-        hipLaunchKernelGGL((k_trace_threaded<kWalkPlain, kVariant>), grid, dim3(block), 0, stream, rays, hits, n, sc,
+        hipLaunchKernelGGL((k_trace_rays<kVariant, false>), grid, dim3(block), lds, stream, rays, hits, n, sc,
                            leaf_batch, counters);
+    return hipGetLastError();
 }
 
 hipError_t launch_trace(const TraceScene& sc, int variant, const TraceRay* rays, TraceHit* hits, uint32_t n,
                         uint32_t block, hipStream_t stream, unsigned long long* counters, const TraceTuning* tune) {
     if (n == 0) return hipSuccess;
-    if (block == 0 && !counters && sc.nnodes != 0) {
-        // persistent kernel: as many resident waves as fit, each with a chunk of the rays
-        const uint32_t cus = tune && tune->cu_count ? tune->cu_count : 256u;
-        // measured on the 1.3M-triangle incoherent set: 7 (stackless) or 8 (threaded) waves per SIMD,
-        // refills at 24 or 48 idle lanes, primitive tests once 12 or 6 lanes wait at leaves. The
-        // stackless walk at 8 waves fetches more from beyond the L2 and is slower: 0.88 ms against
-        // 0.77 (6 waves 0.81)
-        const uint32_t wps = tune && tune->waves_per_simd ? tune->waves_per_simd
-                             : variant == kVariantStackless ? kDefaultWavesStackless : 8u;
-        const uint32_t refill =
-            tune && tune->refill ? tune->refill : (variant != kVariantStackless ? 48u : 24u);
-        const uint32_t leaf_batch = tune && tune->leaf_batch ? tune->leaf_batch
-                                    : variant == kVariantStackless ? kDefaultLeafBatchStackless
-                                                                   : kDefaultLeafBatch;
-        const uint32_t blocks = cus * wps;  // 4 waves (one per SIMD) per 256-thread block
-        const uint32_t waves = blocks * 4u;
-        const uint32_t chunk = (n + waves - 1) / waves;
-        if (variant == kVariantThreaded) {
-            hipLaunchKernelGGL(k_trace_persistent<kVariantThreaded>, dim3(blocks), dim3(256), 0, stream, rays, hits,
-                               n, sc, chunk, refill, leaf_batch, 0u);
-        } else if (variant == kVariantSingleThreaded) {
-            hipLaunchKernelGGL(k_trace_persistent<kVariantSingleThreaded>, dim3(blocks), dim3(256), 0, stream, rays,
-                               hits, n, sc, chunk, refill, leaf_batch, 0u);
-        } else {
-            // the top of the tree in LDS: 128 records (14 KB) beside 8 KB of stacks let the 7
-            // workgroups per CU of the default launch share the CU's 160 KB
-            uint32_t top = tune && tune->treelet ? tune->treelet : kDefaultTreelet;
-            if (top == kTreeletOff) top = 0;
-            top = top < sc.nwalk ? top : sc.nwalk;
-            top = top < kTreeletMaxStaged ? top : kTreeletMaxStaged;
-            hipLaunchKernelGGL(k_trace_persistent<kVariantStackless>, dim3(blocks), dim3(256), walk_lds_bytes(top, 256),
-                               stream, rays, hits, n, sc, chunk, refill, leaf_batch, top);
-        }
+    const TraceTuning t = tune ? *tune : TraceTuning();
+    if (sc.nnodes == 0) {
+        hipLaunchKernelGGL(k_trace_empty, dim3((n + 255) / 256), dim3(256), 0, stream, rays, hits, n);
         return hipGetLastError();
     }
-    if (block == 0) block = 256;
-    dim3 grid((n + block - 1) / block);
-    // one thread per ray: leaves batched by default only once as many lanes wait at leaves as
-    // walk on (leaf_batch 64; leaf_batch 1 asks for the plain walk)
-    const uint32_t leaf_batch = tune && tune->leaf_batch ? tune->leaf_batch : kPerRayLeafBatch;
-    const int mode = counters ? kWalkCount : (leaf_batch > 1 ? kWalkBatched : kWalkPlain);
-    if (sc.nnodes == 0) {
-        hipLaunchKernelGGL(k_trace_empty, grid, dim3(block), 0, stream, rays, hits, n);
-    } else if (variant == kVariantThreaded) {
-        launch_threaded<kVariantThreaded>(mode, grid, block, stream, rays, hits, n, sc, leaf_batch, counters);
-    } else if (variant == kVariantSingleThreaded) {
-        launch_threaded<kVariantSingleThreaded>(mode, grid, block, stream, rays, hits, n, sc, leaf_batch, counters);
-    } else {
-        const size_t lds = walk_lds_bytes(0, block);
-        if (mode == kWalkCount)
-            hipLaunchKernelGGL(k_trace_stackless<true>, grid, dim3(block), lds, stream, rays, hits, n, sc, 1u, counters);
-        else
-            hipLaunchKernelGGL(k_trace_stackless<false>, grid, dim3(block), lds, stream, rays, hits, n, sc, leaf_batch,
-                               counters);
-    }
-    return hipGetLastError();
+    if (variant == kVariantThreaded)
+        return launch_variant<kVariantThreaded>(sc, rays, hits, n, block, stream, counters, t);
+    if (variant == kVariantSingleThreaded)
+        return launch_variant<kVariantSingleThreaded>(sc, rays, hits, n, block, stream, counters, t);
+    return launch_variant<kVariantStackless>(sc, rays, hits, n, block, stream, counters, t);
 }
 
 }  // namespace rgpu

@@ -944,14 +944,13 @@ __device__ __forceinline__ void store_extension(const DevState& s, const TraceSc
 template <int kVariant, class J>
 __global__ void __launch_bounds__(256, 8) k_trace_step(DevState s, WFParams p, J jobs, uint32_t top) {
     const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
-    if constexpr (kVariant == kVariantStackless) {
+    {
         // the top `top` records of the block's scene in LDS (a job owns whole 256-slot blocks,
         // so every slot of a workgroup traces the same scene)
         const uint32_t first = blockIdx.x * blockDim.x;
         const TraceScene sb = jobs.scene(jobs.job(first < p.n ? first : p.n - 1));
-        const uint32_t t = top < sb.nwalk ? top : sb.nwalk;
-        stage_records(reinterpret_cast<const float4*>(sb.walk_nodes), t);
-        top = t;
+        top = top < sb.nwalk ? top : sb.nwalk;
+        stage_records<kVariant>(reinterpret_cast<const float4*>(sb.walk_nodes), top);
     }
     advance_cursors(s, jobs, slot);
     if (slot >= p.n) return;
@@ -1520,16 +1519,17 @@ hipError_t step_impl(const DevState& st, const WFParams& p, const J& jobs, const
             if (e != hipSuccess) return e;
             hipLaunchKernelGGL(k_trace_finish<J>, full, blk, 0, s, st, p, jobs);
         }
-    } else if (variant == kVariantThreaded) {
-        hipLaunchKernelGGL((k_trace_step<kVariantThreaded, J>), tgrid, tblk, 0, s, st, p, jobs, 0u);
-    } else if (variant == kVariantSingleThreaded) {
-        hipLaunchKernelGGL((k_trace_step<kVariantSingleThreaded, J>), tgrid, tblk, 0, s, st, p, jobs, 0u);
     } else {
-        // the top of the tree in LDS: 27 records per wave beside its 2 KB of stacks, so that 8 waves
+        // the top of the tree in LDS: 26 records per wave beside its 2 KB of stacks, so that 8 waves
         // per SIMD fit the 160 KB
-        const uint32_t top = 27u * tb / 64u;
-        hipLaunchKernelGGL((k_trace_step<kVariantStackless, J>), tgrid, tblk, walk_lds_bytes(top, tb), s, st, p, jobs,
-                           top);
+        const uint32_t top = 26u * tb / 64u;
+        const size_t lds = walk_lds_bytes(variant, top, tb);
+        if (variant == kVariantThreaded)
+            hipLaunchKernelGGL((k_trace_step<kVariantThreaded, J>), tgrid, tblk, lds, s, st, p, jobs, top);
+        else if (variant == kVariantSingleThreaded)
+            hipLaunchKernelGGL((k_trace_step<kVariantSingleThreaded, J>), tgrid, tblk, lds, s, st, p, jobs, top);
+        else
+            hipLaunchKernelGGL((k_trace_step<kVariantStackless, J>), tgrid, tblk, lds, s, st, p, jobs, top);
     }
     mark(7);
     hipLaunchKernelGGL(k_logic<J>, full, blk, 0, s, st, p, jobs, g);

@@ -1,6 +1,6 @@
-"""The stackless walk's record form: deep stacks, rays without motion along an axis, odd clips.
+"""The walk records of the ray cast: deep stacks, rays without motion along an axis, odd clips.
 
-Bit-exact against the oracle's binary walk on the same tree, as the other traversal tests: the
+Bit-exact against the oracle's binary walks on the same tree, as the other traversal tests: the
 walk takes two tree levels a visit, keeps what it defers in LDS and then in private memory, and
 visits binary nodes one by one where a wave's rays allow nothing else.
 """
@@ -19,10 +19,19 @@ SAME = dict(prim=0, t=0, uv=0)
 def _check(ctx, v, f, rays, sph=None, **opt):
     bvh = _lib.BVH(v, f, sph, **opt)
     scene = _lib.Scene(ctx, bvh)
-    o, _ = O.intersect_stackless(O.RefStackless(bvh.export()), v, f, rays, sph)
-    for block in (0, 64, 256):
-        g = _lib.trace(ctx, scene, rays, "stackless", block=block)
-        assert H.compare_hits(g, o) == SAME, (block, bvh.depth)
+    tree = bvh.export()
+    for variant in ("stackless", "threaded", "threaded_single"):
+        if variant == "stackless":
+            o, cnt = O.intersect_stackless(O.RefStackless(tree), v, f, rays, sph)
+        elif variant == "threaded":
+            o, cnt = O.intersect_mtbvh(O.RefMTBVH(tree), v, f, rays, sph)
+        else:
+            o, cnt = O.intersect_tbvh(O.RefMTBVH(tree), v, f, rays, sph)
+        for block in (0, 64, 256):
+            g = _lib.trace(ctx, scene, rays, variant, block=block)
+            assert H.compare_hits(g, o) == SAME, (variant, block, bvh.depth)
+        rd, hd = ctx.to_device(rays), ctx.alloc(len(rays) * 16)
+        assert scene.extension_ray_cast_stats(variant, rd, hd, len(rays)) == cnt, variant
     scene.close()
     return bvh
 
