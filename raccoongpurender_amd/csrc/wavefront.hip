@@ -438,10 +438,10 @@ __global__ void __launch_bounds__(256) k_clear_accum(DevState s, uint32_t npixel
 // paths (its queue position less the job's first position, the scanned offset of its first
 // block); a job past its sample budget parks the slot (pixel kDeadPixel, in no queue).
 template <class J>
-__global__ void __launch_bounds__(256) k_new_path(DevState s, WFParams p, J jobs, DevGuide g) {
-    const uint32_t count = s.counts[0];
+__device__ __forceinline__ void new_path_item(uint32_t i, const DevState& s, const WFParams& p, const J& jobs,
+                                              const DevGuide& g) {
     const unsigned long long base0 = J::kBatch ? 0ull : *s.next_pixel;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
+    {
         const uint32_t slot = s.items[i];
         const uint32_t jb = jobs.job(slot);
         const Camera& cam = jobs.camera(jb);
@@ -452,7 +452,7 @@ __global__ void __launch_bounds__(256) k_new_path(DevState s, WFParams p, J jobs
             sample = jd.next_pixel + (i - s.block_counts[jd.first_block]);
             if (jd.budget != 0 && sample >= jd.budget) {
                 store_ray_rec(s.ray, slot, F3{0.0f, 0.0f, 0.0f}, -1.0f, F3{0.0f, 0.0f, 1.0f}, kDeadPixel);
-                continue;
+                return;
             }
         }
         const unsigned long long P = (unsigned long long)cam.width * cam.height;
@@ -497,7 +497,7 @@ __global__ void __launch_bounds__(256) k_new_path(DevState s, WFParams p, J jobs
     }
 }
 
-__device__ __forceinline__ void spawn(DevState& s, uint32_t slot, F3 ro, F3 rd, float t, F3 wi, F3 ng_offset,
+__device__ __forceinline__ void spawn(const DevState& s, uint32_t slot, F3 ro, F3 rd, float t, F3 wi, F3 ng_offset,
                                       bool offset_normal, uint32_t pixel) {
     // ro + rd * tmin + wi * 1e-5 (+ Ng * 1e-5)  (kernels/lambertian.cl:117-119)
     F3 o = add3(add3(ro, mul3(rd, t)), mul3(wi, 1.0e-5f));
@@ -545,10 +545,10 @@ __device__ __forceinline__ void record_vertex(const DevGuide& g, const GuideFram
 // Lambertian: strategy selection + envmap 6-axis sample / cosine sample + pdfs +
 // lambertian_stage (mixture_density.cl, envmap_sampling.cl:169-217,250-266, lambertian.cl:34-123).
 template <bool kGuided, class J>
-__global__ void __launch_bounds__(256) k_shade_lambertian(DevState s, WFParams p, J jobs, DevGuide g) {
-    const uint32_t count = s.counts[kMatLambertian];
+__device__ __forceinline__ void lambertian_item(uint32_t i, const DevState& s, const WFParams& p, const J& jobs,
+                                        const DevGuide& g) {
     const uint32_t* items = s.items + (size_t)kMatLambertian * p.n;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
+    {
         const uint32_t slot = items[i];
         const uint32_t jb = jobs.job(slot);
         const DevMaterials m = jobs.mats(jb);
@@ -629,10 +629,10 @@ __global__ void __launch_bounds__(256) k_shade_lambertian(DevState s, WFParams p
 
 // Ward (mixture_density.cl, envmap_sampling.cl, ward.cl:76-186)
 template <bool kGuided, class J>
-__global__ void __launch_bounds__(256) k_shade_ward(DevState s, WFParams p, J jobs, DevGuide g) {
-    const uint32_t count = s.counts[kMatWard];
+__device__ __forceinline__ void ward_item(uint32_t i, const DevState& s, const WFParams& p, const J& jobs,
+                                        const DevGuide& g) {
     const uint32_t* items = s.items + (size_t)kMatWard * p.n;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
+    {
         const uint32_t slot = items[i];
         const uint32_t jb = jobs.job(slot);
         const DevMaterials m = jobs.mats(jb);
@@ -709,10 +709,9 @@ __global__ void __launch_bounds__(256) k_shade_ward(DevState s, WFParams p, J jo
 }
 
 // Mirror (kernels/delta_materials.cl:48-77)
-__global__ void __launch_bounds__(256) k_shade_specular(DevState s, WFParams p) {
-    const uint32_t count = s.counts[kMatSpecular];
+__device__ __forceinline__ void specular_item(uint32_t i, const DevState& s, const WFParams& p) {
     const uint32_t* items = s.items + (size_t)kMatSpecular * p.n;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
+    {
         const uint32_t slot = items[i];
         uint4 st = s.rng[slot];
         ExtRec e = s.ext[slot];
@@ -731,10 +730,9 @@ __global__ void __launch_bounds__(256) k_shade_specular(DevState s, WFParams p) 
 
 // Dielectric (kernels/delta_materials.cl:79-134)
 template <class J>
-__global__ void __launch_bounds__(256) k_shade_dielectric(DevState s, WFParams p, J jobs) {
-    const uint32_t count = s.counts[kMatDielectric];
+__device__ __forceinline__ void dielectric_item(uint32_t i, const DevState& s, const WFParams& p, const J& jobs) {
     const uint32_t* items = s.items + (size_t)kMatDielectric * p.n;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
+    {
         const uint32_t slot = items[i];
         const DevMaterials m = jobs.mats(jobs.job(slot));
         uint4 st = s.rng[slot];
@@ -789,10 +787,9 @@ __device__ __forceinline__ uint32_t volume_hash(const Volume& v) {
 
 // Medium boundary (kernels/homogeneous_volume.cl:19-64, InVolumeList ops types.cl:108-132)
 template <class J>
-__global__ void __launch_bounds__(256) k_shade_volume_surface(DevState s, WFParams p, J jobs) {
-    const uint32_t count = s.counts[kMatVolume];
+__device__ __forceinline__ void volume_surface_item(uint32_t i, const DevState& s, const WFParams& p, const J& jobs) {
     const uint32_t* items = s.items + (size_t)kMatVolume * p.n;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
+    {
         const uint32_t slot = items[i];
         const DevMaterials m = jobs.mats(jobs.job(slot));
         uint4 st = s.rng[slot];
@@ -827,10 +824,9 @@ __global__ void __launch_bounds__(256) k_shade_volume_surface(DevState s, WFPara
 // Scattering inside a medium (mixture_density.cl:47-51, envmap_sampling.cl:219-248,268-281,
 // homogeneous_volume.cl:66-129)
 template <class J>
-__global__ void __launch_bounds__(256) k_shade_volume_inside(DevState s, WFParams p, J jobs) {
-    const uint32_t count = s.counts[kMatVolumeInside];
+__device__ __forceinline__ void volume_inside_item(uint32_t i, const DevState& s, const WFParams& p, const J& jobs) {
     const uint32_t* items = s.items + (size_t)kMatVolumeInside * p.n;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
+    {
         const uint32_t slot = items[i];
         const uint32_t jb = jobs.job(slot);
         const DevMaterials m = jobs.mats(jb);
@@ -865,6 +861,42 @@ __global__ void __launch_bounds__(256) k_shade_volume_inside(DevState s, WFParam
         store_shade(s.shade, slot, F3{0.0f, 0.0f, 0.0f}, T);
         store_ray_rec(s.ray, slot, add3(ro, mul3(rd, e.tmin)), kFltMax, wi, pixel);
         s.rng[slot] = st;
+    }
+}
+
+// The stage queues of a bounce in one launch (kQueues: one bit per queue): workgroups of 256 items,
+// one queue's after another's, found from the queue lengths on the device; a grid smaller than
+// the work strides over it. A slot is in one queue, so the stages are independent.
+// Seven launches (a queue each) cost about 4.5 us apiece however short their queues, and a large
+// bounce drained the chip seven times. In one launch, whose items differ in what bounds them
+// (scattered records, or the Ward terms' double-precision arithmetic), a bounce of 4,096 slots
+// takes 69 us instead of 91, of 2^18 (small scene, every material) 111 instead of 137, of 2^20
+// 263 instead of 283, of 2^22 (1080p workload) 1.98 ms instead of 2.02. The kernel holds the
+// largest stage's registers (107); held to 5 or 6 waves per SIMD it is 1 and 2 % slower.
+constexpr uint32_t kAllQueues = (1u << kNumQueues) - 1u;
+template <uint32_t kQueues, bool kGuided, class J>
+__global__ void __launch_bounds__(256) k_shade(DevState s, WFParams p, J jobs, DevGuide g) {
+    for (uint32_t block = blockIdx.x;; block += gridDim.x) {
+        uint32_t b = block;
+        int q = 0;
+        uint32_t count = 0;
+        for (; q < kNumQueues; ++q) {
+            if (!((kQueues >> q) & 1u)) continue;
+            count = s.counts[q];
+            const uint32_t blocks = (count + 255u) / 256u;
+            if (b < blocks) break;
+            b -= blocks;
+        }
+        if (q == kNumQueues) return;
+        const uint32_t i = b * 256u + threadIdx.x;
+        if (i >= count) continue;
+        if ((kQueues & 1u) && q == 0) new_path_item(i, s, p, jobs, g);
+        else if ((kQueues >> kMatLambertian & 1u) && q == kMatLambertian) lambertian_item<kGuided>(i, s, p, jobs, g);
+        else if ((kQueues >> kMatWard & 1u) && q == kMatWard) ward_item<kGuided>(i, s, p, jobs, g);
+        else if ((kQueues >> kMatSpecular & 1u) && q == kMatSpecular) specular_item(i, s, p);
+        else if ((kQueues >> kMatDielectric & 1u) && q == kMatDielectric) dielectric_item(i, s, p, jobs);
+        else if ((kQueues >> kMatVolume & 1u) && q == kMatVolume) volume_surface_item(i, s, p, jobs);
+        else if (kQueues >> kMatVolumeInside & 1u) volume_inside_item(i, s, p, jobs);
     }
 }
 
@@ -1488,27 +1520,35 @@ hipError_t step_impl(const DevState& st, const WFParams& p, const J& jobs, const
         if (marks) (void)hipEventRecord(marks[k], s);
     };
     mark(0);
-    hipLaunchKernelGGL(k_new_path<J>, qgrid, blk, 0, s, st, p, jobs, g);
-    mark(1);
-    if (g.enabled) {
+    const uint32_t need = (p.n + 255u) / 256u + (uint32_t)kNumQueues;  // every queue's last block may be partial
+    const dim3 sgrid(need < qgrid.x ? need : qgrid.x);
+    if (marks) {
+        // between marks each stage is a launch of its own
+        hipLaunchKernelGGL((k_shade<1u, false, J>), sgrid, blk, 0, s, st, p, jobs, g);
+        mark(1);
+        if (g.enabled) {
+            hipError_t e = guide_infer(st, p, g, jobs.table(), s);
+            if (e != hipSuccess) return e;
+        }
+        mark(2);
+        if (g.enabled) hipLaunchKernelGGL((k_shade<1u << kMatLambertian, true, J>), sgrid, blk, 0, s, st, p, jobs, g);
+        else hipLaunchKernelGGL((k_shade<1u << kMatLambertian, false, J>), sgrid, blk, 0, s, st, p, jobs, g);
+        mark(3);
+        if (g.enabled) hipLaunchKernelGGL((k_shade<1u << kMatWard, true, J>), sgrid, blk, 0, s, st, p, jobs, g);
+        else hipLaunchKernelGGL((k_shade<1u << kMatWard, false, J>), sgrid, blk, 0, s, st, p, jobs, g);
+        mark(4);
+        hipLaunchKernelGGL((k_shade<1u << kMatSpecular | 1u << kMatDielectric, false, J>), sgrid, blk, 0, s, st, p,
+                           jobs, g);
+        mark(5);
+        hipLaunchKernelGGL((k_shade<1u << kMatVolume | 1u << kMatVolumeInside, false, J>), sgrid, blk, 0, s, st, p,
+                           jobs, g);
+    } else if (g.enabled) {
         hipError_t e = guide_infer(st, p, g, jobs.table(), s);
         if (e != hipSuccess) return e;
-        mark(2);
-        hipLaunchKernelGGL((k_shade_lambertian<true, J>), qgrid, blk, 0, s, st, p, jobs, g);
-        mark(3);
-        hipLaunchKernelGGL((k_shade_ward<true, J>), qgrid, blk, 0, s, st, p, jobs, g);
+        hipLaunchKernelGGL((k_shade<kAllQueues, true, J>), sgrid, blk, 0, s, st, p, jobs, g);
     } else {
-        mark(2);
-        hipLaunchKernelGGL((k_shade_lambertian<false, J>), qgrid, blk, 0, s, st, p, jobs, g);
-        mark(3);
-        hipLaunchKernelGGL((k_shade_ward<false, J>), qgrid, blk, 0, s, st, p, jobs, g);
+        hipLaunchKernelGGL((k_shade<kAllQueues, false, J>), sgrid, blk, 0, s, st, p, jobs, g);
     }
-    mark(4);
-    hipLaunchKernelGGL(k_shade_specular, qgrid, blk, 0, s, st, p);
-    hipLaunchKernelGGL(k_shade_dielectric<J>, qgrid, blk, 0, s, st, p, jobs);
-    mark(5);
-    hipLaunchKernelGGL(k_shade_volume_surface<J>, qgrid, blk, 0, s, st, p, jobs);
-    hipLaunchKernelGGL(k_shade_volume_inside<J>, qgrid, blk, 0, s, st, p, jobs);
     mark(6);
     // trace_block 0: a single render casts through the persistent ray-cast kernel; a batch (several
     // scenes) keeps one thread per slot (tgrid is 256 wide then)
