@@ -9,6 +9,8 @@
 // invariants (each primitive in exactly one leaf, children inside parents, depth).
 #include "bvh_build.h"
 
+#include "fingerprint.h"
+
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
@@ -372,95 +374,11 @@ void mark_leaf_links(std::vector<SLNode>* nodes) {
     }
 }
 
-uint32_t pack_walk(const BVHTree& t, uint32_t top, std::vector<WalkNode>* out) {
-    const std::vector<BuildNode>& nodes = t.nodes;
-    const size_t nn = nodes.size();
-    out->clear();
-    if (nn == 0) return kInvalid;
-    auto branch = [&](int32_t i) { return nodes[i].left >= 0; };
-    auto word = [&](int32_t i) {
-        return kLeafFlag | ((nodes[i].prim_cnt - 1) << 28) | nodes[i].prim_beg;
-    };
-    if (!branch(0)) return word(0);
-    // the grandchildren of a record's node, the children of a leaf child being itself
-    auto family = [&](int32_t i, int32_t g[4]) {
-        const int32_t kids[2] = {nodes[i].left, nodes[i].right};
-        for (int k = 0; k < 2; ++k) {
-            g[2 * k] = branch(kids[k]) ? nodes[kids[k]].left : kids[k];
-            g[2 * k + 1] = branch(kids[k]) ? nodes[kids[k]].right : kids[k];
-        }
-    };
-    // parents precede their children in the tree's order: depth parity, then the ids
-    std::vector<uint8_t> odd(nn, 0);
-    std::vector<uint32_t> id(nn, kInvalid);
-    std::vector<int32_t> order;  // record id -> node
-    for (size_t i = 0; i < nn; ++i)
-        if (branch((int32_t)i)) odd[nodes[i].left] = odd[nodes[i].right] = odd[i] ^ 1;
-    order.push_back(0);
-    id[0] = 0;
-    for (size_t h = 0; h < order.size() && order.size() < top; ++h) {
-        int32_t g[4];
-        family(order[h], g);
-        for (int k = 0; k < 4 && order.size() < top; ++k)
-            if (branch(g[k]) && !odd[g[k]] && id[g[k]] == kInvalid) {
-                id[g[k]] = (uint32_t)order.size();
-                order.push_back(g[k]);
-            }
-    }
-    for (size_t i = 0; i < nn; ++i)
-        if (!odd[i] && id[i] == kInvalid && branch((int32_t)i)) {
-            id[i] = (uint32_t)order.size();
-            order.push_back((int32_t)i);
-        }
-    // Whether a branch's right child comes first, a bit per direction class. The six direction
-    // sorts are applied one after another to the same tree, as common/threaded_bvh.hpp:518-525
-    // does, so a child pair whose centres tie is swapped by every sort.
-    auto orders = [&](int32_t i) {
-        uint32_t bits = 0;
-        bool swapped = false;
-        for (int dir = 0; branch(i) && dir < 6; ++dir) {
-            const BuildNode& a = nodes[swapped ? nodes[i].right : nodes[i].left];
-            const BuildNode& b = nodes[swapped ? nodes[i].left : nodes[i].right];
-            const int axis = dir / 2;
-            float lc = 0.5f * (a.bmin[axis] + a.bmax[axis]);
-            float rc = 0.5f * (b.bmin[axis] + b.bmax[axis]);
-            if (dir & 1) std::swap(lc, rc);
-            if (!(lc < rc)) swapped = !swapped;
-            bits |= (swapped ? 1u : 0u) << dir;
-        }
-        return bits;
-    };
-    out->resize(order.size());
-    for (size_t r = 0; r < order.size(); ++r) {
-        WalkNode& w = (*out)[r];
-        const uint32_t o[3] = {orders(order[r]), orders(nodes[order[r]].left), orders(nodes[order[r]].right)};
-        w.order = 0;
-        for (int dir = 0; dir < 6; ++dir)
-            for (int k = 0; k < 3; ++k) w.order |= ((o[k] >> dir) & 1u) << (3 * dir + k);
-        int32_t g[4];
-        family(order[r], g);
-        for (int k = 0; k < 4; ++k) {
-            for (int a = 0; a < 3; ++a) {
-                w.box[k][a] = nodes[g[k]].bmin[a];
-                w.box[k][3 + a] = nodes[g[k]].bmax[a];
-            }
-            w.link[k] = branch(g[k]) ? 8 * id[g[k]] : word(g[k]);
-        }
-        for (uint32_t& x : w.pad) x = 0;
-        for (int k = 0; k < 4; k += 2)
-            if (g[k] == g[k + 1]) w.link[k + 1] = kInvalid;  // a leaf child
-    }
-    return 0;
-}
-
-void pack_prims(const BVHTree& t, const float* points, uint32_t stride,
-                const uint32_t* indices, uint32_t ntris,
-                const float* spheres, uint32_t nspheres, std::vector<PrimRec>* out) {
-    (void)nspheres;
-    out->assign(t.prim_ids.size(), PrimRec());
-    for (size_t s = 0; s < t.prim_ids.size(); ++s) {
-        uint32_t p = t.prim_ids[s];
-        PrimRec& r = (*out)[s];
+void pack_prims(const BVHTree& t, const float* points, uint32_t stride, const uint32_t* indices, uint32_t ntris,
+                const float* spheres, size_t first, size_t count, PrimRec* out) {
+    for (size_t s = 0; s < count; ++s) {
+        const uint32_t p = t.prim_ids[first + s];
+        PrimRec& r = out[s];
         std::memset(&r, 0, sizeof(r));
         r.prim = p;
         if (p < ntris) {
@@ -480,6 +398,101 @@ void pack_prims(const BVHTree& t, const float* points, uint32_t stride,
             r.q0[0] = sp[0]; r.q0[1] = sp[1]; r.q0[2] = sp[2]; r.q0[3] = sp[3];
         }
     }
+}
+
+namespace {
+// Pieces 0..count-1 made by make(piece, buffer), a few at a time on threads of their own, and
+// added to f in order, each while the next ones are being made.
+template <class T, class Make>
+void add_pieces(Fingerprint* f, size_t count, uint32_t threads, Make make) {
+    const size_t width = std::max<size_t>(1, std::min<size_t>(threads, count));
+    std::vector<std::vector<T>> ready(width), next(width);
+    size_t made = 0;  // pieces in `ready`
+    for (size_t at = 0; at < count || made != 0;) {
+        const size_t n = std::min(width, count - at);
+        std::vector<std::future<void>> jobs;
+        for (size_t j = 0; j < n; ++j) {
+            if (width == 1) make(at + j, &next[j]);
+            else jobs.push_back(std::async(std::launch::async, [&, j] { make(at + j, &next[j]); }));
+        }
+        for (size_t j = 0; j < made; ++j)
+            if (!ready[j].empty()) f->add(ready[j].data(), ready[j].size() * sizeof(T));
+        for (std::future<void>& job : jobs) job.get();
+        ready.swap(next);
+        made = n;
+        at += n;
+    }
+}
+}  // namespace
+
+uint64_t scene_fingerprint(const BVHTree& t, uint32_t top, const float* points, uint32_t stride,
+                           const uint32_t* indices, uint32_t ntris, const float* spheres, uint32_t threads) {
+    const std::vector<BuildNode>& nodes = t.nodes;
+    const size_t nn = nodes.size();
+    // number_top_breadth_first's order: the first `top` nodes breadth-first, the others as they are
+    std::vector<uint32_t> order;
+    if (nn) order.push_back(0);
+    for (size_t h = 0; h < order.size() && order.size() < top; ++h) {
+        const BuildNode& b = nodes[order[h]];
+        if (b.left < 0) continue;
+        order.push_back((uint32_t)b.left);
+        if (order.size() < top) order.push_back((uint32_t)b.right);
+    }
+    std::vector<uint32_t> id(nn, kInvalid), parent(nn, 0);
+    for (size_t k = 0; k < order.size(); ++k) id[order[k]] = (uint32_t)k;
+    uint32_t given = (uint32_t)order.size();
+    for (size_t i = 0; i < nn; ++i) {
+        if (id[i] == kInvalid) id[i] = given++;
+        if (nodes[i].left >= 0) parent[nodes[i].left] = parent[nodes[i].right] = (uint32_t)i;
+    }
+    auto marked = [&](uint32_t i) { return id[i] | (nodes[i].left < 0 ? kChildLeaf : 0u); };
+    auto record = [&](uint32_t i) {
+        SLNode s;
+        std::memset(&s, 0, sizeof(s));
+        const BuildNode& b = nodes[i];
+        if (b.left >= 0) {
+            const BuildNode &l = nodes[b.left], &r = nodes[b.right];
+            for (int k = 0; k < 3; ++k) {
+                s.lmin[k] = l.bmin[k];
+                s.lmax[k] = l.bmax[k];
+                s.rmin[k] = r.bmin[k];
+                s.rmax[k] = r.bmax[k];
+            }
+            s.a = marked((uint32_t)b.left);
+            s.b = marked((uint32_t)b.right);
+        } else {
+            s.a = kLeafFlag | b.prim_beg;
+            s.b = b.prim_beg + b.prim_cnt;
+        }
+        if (i != 0) {  // the root has neither
+            const BuildNode& p = nodes[parent[i]];
+            s.parent = id[parent[i]];
+            s.sibling = marked((uint32_t)((uint32_t)p.left == i ? p.right : p.left));
+        }
+        return s;
+    };
+    const size_t kPiece = 16384;  // 1 MB of node records
+    Fingerprint f(ntris);
+    if (nn) {
+        std::vector<SLNode> head;
+        for (const uint32_t i : order) head.push_back(record(i));
+        f.add(head.data(), head.size() * sizeof(SLNode));
+    }
+    std::vector<uint8_t> first(nn, 0);  // nodes of the head
+    for (const uint32_t i : order) first[i] = 1;
+    add_pieces<SLNode>(&f, (nn + kPiece - 1) / kPiece, threads, [&](size_t piece, std::vector<SLNode>* out) {
+        out->clear();
+        for (size_t i = piece * kPiece; i < std::min(nn, (piece + 1) * kPiece); ++i)
+            if (!first[i]) out->push_back(record((uint32_t)i));
+    });
+    Fingerprint g(f.value());
+    const size_t slots = t.prim_ids.size();
+    add_pieces<PrimRec>(&g, (slots + kPiece - 1) / kPiece, threads, [&](size_t piece, std::vector<PrimRec>* out) {
+        const size_t beg = piece * kPiece, n = std::min(slots, beg + kPiece) - beg;
+        out->resize(n);
+        pack_prims(t, points, stride, indices, ntris, spheres, beg, n, out->data());
+    });
+    return g.value();
 }
 
 }  // namespace rgpu

@@ -1,5 +1,6 @@
 // Host-side BVH construction and packing into the device layouts of rgpu_types.h.
 #pragma once
+#include <stddef.h>
 #include <stdint.h>
 #include <vector>
 #include "rgpu_types.h"
@@ -49,12 +50,13 @@ void pack_stackless(const BVHTree& t, std::vector<SLNode>* out);
 void number_top_breadth_first(std::vector<SLNode>* nodes, uint32_t top);
 // Sets kChildLeaf on the child and sibling ids that name leaves (after any renumbering).
 void mark_leaf_links(std::vector<SLNode>* nodes);
-// Records of the device's walk: the first `top` in breadth-first order (so that any LDS
-// copy of the top of the tree is a prefix), the others in the tree's depth-first order. Returns
-// the root's link.
-uint32_t pack_walk(const BVHTree& t, uint32_t top, std::vector<WalkNode>* out);
-void pack_prims(const BVHTree& t, const float* points, uint32_t stride,
-                const uint32_t* indices, uint32_t ntris,
-                const float* spheres, uint32_t nspheres, std::vector<PrimRec>* out);
+// Primitive records of the slots [first, first + count).
+void pack_prims(const BVHTree& t, const float* points, uint32_t stride, const uint32_t* indices, uint32_t ntris,
+                const float* spheres, size_t first, size_t count, PrimRec* out);
+// Fingerprint of a scene: of its stackless records as pack_stackless, number_top_breadth_first(top)
+// and mark_leaf_links give them, seeded with ntris, then of its primitive records seeded with that.
+// The records are made piece by piece, by up to `threads` threads, and never held as a whole.
+uint64_t scene_fingerprint(const BVHTree& t, uint32_t top, const float* points, uint32_t stride,
+                           const uint32_t* indices, uint32_t ntris, const float* spheres, uint32_t threads);
 
 }  // namespace rgpu

@@ -27,4 +27,9 @@ void build_bvh_device(const float* points, uint32_t stride, uint32_t npoints, co
                       uint32_t ntris, const float* spheres, uint32_t nspheres, const BuildOptions& opt,
                       hipStream_t s, BVHTree* out, BuildTimes* times);
 
+// Exclusive prefix sum on stream s: out[i] = in[0] + .. + in[i-1] for i < n; tmp: scan_temp_words(n)
+// words.
+size_t scan_temp_words(size_t n);
+hipError_t scan_exclusive(const uint32_t* in, uint32_t* out, size_t n, uint32_t* tmp, hipStream_t s);
+
 }  // namespace rgpu

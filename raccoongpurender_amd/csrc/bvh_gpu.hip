@@ -888,6 +888,8 @@ __global__ void k_scan_add(uint32_t* __restrict__ out, size_t n, const uint32_t*
     if (i < n) out[i] += offs[i / kScanPer];
 }
 
+}  // namespace
+
 size_t scan_temp_words(size_t n) {
     size_t w = 0;
     while (n > kScanPer) {
@@ -897,7 +899,6 @@ size_t scan_temp_words(size_t n) {
     return w + 2;
 }
 
-// out[i] = sum of in[0..i) for i < n; tmp: scan_temp_words(n) words.
 hipError_t scan_exclusive(const uint32_t* in, uint32_t* out, size_t n, uint32_t* tmp, hipStream_t s) {
     const size_t nb = (n + kScanPer - 1) / kScanPer;
     uint32_t* sums = tmp;
@@ -911,6 +912,7 @@ hipError_t scan_exclusive(const uint32_t* in, uint32_t* out, size_t n, uint32_t*
     return hipGetLastError();
 }
 
+namespace {
 // ------------------------------------------------------------------ host driver
 // A pair of events owned for the span of one build.
 struct Events {

@@ -12,12 +12,12 @@
 #include <new>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/raccoon_gpu.h"
 #include "bvh_build.h"
 #include "bvh_gpu.h"
-#include "fingerprint.h"
 #include "rgpu_traverse.h"
 #include "rgpu_ctx.h"
 #include "rgpu_scene.h"
@@ -318,23 +318,10 @@ int rgpu_bvh_export(const rgpu_bvh* bvh, float* bounds, int32_t* left, int32_t* 
 }
 
 // ------------------------------------------------------------------ scene
-static int upload_new(rgpu_ctx* ctx, const void* src, size_t bytes, void** dst) {
-    *dst = nullptr;
-    if (bytes == 0) return RGPU_OK;
-    RGPU_HIP(ctx, hipMalloc(dst, bytes));
-    hipError_t e = hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        (void)hipFree(*dst);
-        *dst = nullptr;
-        return hip_fail(ctx, e, "hipMemcpy(scene upload)");
-    }
-    return RGPU_OK;
-}
-
 int rgpu_scene_destroy(rgpu_scene* s) {
     if (!s) return RGPU_ERR_INVALID_ARG;
     if (s->ctx) (void)hipSetDevice(s->ctx->device);
-    for (void* p : {s->walk, s->prims, s->points, s->indices, s->spheres})
+    for (void* p : {s->tables.walk, s->tables.prims, s->tables.points, s->tables.indices, s->tables.spheres})
         if (p) (void)hipFree(p);
     delete s;
     return RGPU_OK;
@@ -353,58 +340,39 @@ int rgpu_scene_create(rgpu_ctx* ctx, const rgpu_bvh* bvh, const float* points, u
         return fail(ctx, RGPU_ERR_INVALID_ARG, "BVH has 2^30 nodes or more");
     RGPU_GUARD_BEGIN
     RGPU_HIP(ctx, hipSetDevice(ctx->device));
-    std::vector<SLNode> sl;
-    std::vector<PrimRec> pr;
-    std::vector<WalkNode> walk;
-    // beside the other packers (its future waits for it on every way out)
-    std::future<uint32_t> packed =
-        std::async(std::launch::async, [&] { return pack_walk(bvh->tree, kTreeletMaxNodes, &walk); });
-    pack_stackless(bvh->tree, &sl);
-    number_top_breadth_first(&sl, kTreeletMaxNodes);
-    mark_leaf_links(&sl);
-    const uint64_t sl_print = fingerprint64(sl.data(), sl.size() * sizeof(SLNode), ntris);
-    pack_prims(bvh->tree, points, stride, indices, ntris, spheres, nspheres, &pr);
-    std::vector<float> p4((size_t)npoints * 4, 0.0f);
-    for (uint32_t i = 0; i < npoints; ++i)
-        for (int k = 0; k < 3; ++k) p4[4 * (size_t)i + k] = points[(size_t)i * stride + k];
-    const uint32_t root = packed.get();
+    uint32_t most = 0;  // the packing kernels read the vertices by these
+    for (size_t i = 0; i < 3 * (size_t)ntris; ++i) most = std::max(most, indices[i]);
+    if (ntris && most >= npoints) return fail(ctx, RGPU_ERR_INVALID_ARG, "triangle index out of range");
+    // the fingerprint's host work runs beside the upload and the packing kernels (its future waits
+    // for it on every way out)
+    const uint32_t threads = std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
+    std::future<uint64_t> print = std::async(std::launch::async, [&] {
+        return scene_fingerprint(bvh->tree, kTreeletMaxNodes, points, stride, indices, ntris, spheres, threads);
+    });
     rgpu_scene* s = new rgpu_scene();
     s->ctx = ctx;
-    int rc = RGPU_OK;
-    if (rc == RGPU_OK) rc = upload_new(ctx, walk.data(), walk.size() * sizeof(WalkNode), &s->walk);
-    if (rc == RGPU_OK) rc = upload_new(ctx, pr.data(), pr.size() * sizeof(PrimRec), &s->prims);
-    if (rc == RGPU_OK) rc = upload_new(ctx, p4.data(), p4.size() * sizeof(float), &s->points);
-    if (rc == RGPU_OK) rc = upload_new(ctx, indices, (size_t)ntris * 3 * sizeof(uint32_t), &s->indices);
-    if (rc == RGPU_OK) rc = upload_new(ctx, spheres, (size_t)nspheres * 4 * sizeof(float), &s->spheres);
-    if (rc != RGPU_OK) {
+    const hipError_t e = pack_scene(bvh->tree, points, stride, npoints, indices, ntris, spheres, nspheres, ctx->stream,
+                                    &s->tables, &s->dev);
+    if (e != hipSuccess) {
         rgpu_scene_destroy(s);
-        return rc;
+        return hip_fail(ctx, e, "rgpu_scene_create");
     }
-    s->dev.walk_nodes = (const WalkNode*)s->walk;
-    s->dev.nwalk = (uint32_t)walk.size();
-    s->dev.prims = (const PrimRec*)s->prims;
-    s->dev.points = (const float4*)s->points;
-    s->dev.indices = (const uint32_t*)s->indices;
-    s->dev.spheres = (const float4*)s->spheres;
-    s->dev.root = root;
-    s->dev.nnodes = (uint32_t)bvh->tree.nodes.size();
-    s->dev.sphere_begin = (int32_t)ntris;
-    bool finite = true;
-    for (const BuildNode& b : bvh->tree.nodes)
-        for (int k = 0; k < 3; ++k)
-            finite = finite && std::isfinite(b.bmin[k]) && std::isfinite(b.bmax[k]) && b.bmin[k] <= b.bmax[k];
-    s->dev.boxes_finite = finite ? 1u : 0u;
+    try {
+        s->fingerprint = print.get();
+    } catch (...) {
+        rgpu_scene_destroy(s);
+        throw;
+    }
     s->nprims = ntris + nspheres;
-    s->fingerprint = fingerprint64(pr.data(), pr.size() * sizeof(PrimRec), sl_print);
     if (!bvh->tree.nodes.empty())
         for (int k = 0; k < 3; ++k) {
-            s->lo[k] = s->dev.root_lo[k] = bvh->tree.nodes[0].bmin[k];
-            s->hi[k] = s->dev.root_hi[k] = bvh->tree.nodes[0].bmax[k];
+            s->lo[k] = bvh->tree.nodes[0].bmin[k];
+            s->hi[k] = bvh->tree.nodes[0].bmax[k];
         }
-    s->bytes[0] = walk.size() * sizeof(WalkNode);
+    s->bytes[0] = (uint64_t)s->dev.nwalk * sizeof(WalkNode);
     s->bytes[1] = 0;  // the threaded walks' child orders are bits of the walk records
-    s->bytes[2] = pr.size() * sizeof(PrimRec);
-    s->bytes[3] = p4.size() * sizeof(float) + (size_t)ntris * 12 + (size_t)nspheres * 16;
+    s->bytes[2] = (uint64_t)s->nprims * sizeof(PrimRec);
+    s->bytes[3] = (uint64_t)npoints * 16 + (uint64_t)ntris * 12 + (uint64_t)nspheres * 16;
     *out = s;
     return RGPU_OK;
     RGPU_GUARD_END(ctx)

@@ -4,15 +4,12 @@
 
 #include "rgpu_ctx.h"
 #include "rgpu_traverse.h"
+#include "scene_pack.h"
 
 struct rgpu_scene {
     rgpu_ctx* ctx = nullptr;
     rgpu::TraceScene dev;
-    void* walk = nullptr;
-    void* prims = nullptr;
-    void* points = nullptr;
-    void* indices = nullptr;
-    void* spheres = nullptr;
+    rgpu::SceneTables tables;
     uint32_t nprims = 0;  // triangles + spheres
     uint64_t fingerprint = 0;  // of the packed node and primitive records (checkpoints compare it)
     uint64_t bytes[4] = {0, 0, 0, 0};

@@ -1,0 +1,279 @@
+// Scene tables packed on the device (rgpu_scene_create; common/scene_manager.hpp:579-591).
+//
+// Bound: the upload of the tree and the geometry over PCIe (70 B per triangle). Packing on the
+// host took one thread 25 ms for the primitive records of 1.3M triangles, as much again for the
+// walk records, and uploaded both tables (112 MB); here the kernels read the uploaded tree (40 B a
+// node) and geometry from HBM and write the tables in place, about 0.2 ms in all.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <algorithm>
+#include <vector>
+
+#include "bvh_gpu.h"
+#include "scene_pack.h"
+
+namespace rgpu {
+namespace {
+
+constexpr uint32_t kNone = 0xFFFFFFFFu;
+
+__device__ __forceinline__ bool is_branch(const BuildNode& n) { return n.left >= 0; }
+__device__ __forceinline__ uint32_t leaf_word(const BuildNode& n) {
+    return kLeafFlag | ((n.prim_cnt - 1u) << 28) | n.prim_beg;
+}
+
+__global__ void __launch_bounds__(256) k_parents(const BuildNode* __restrict__ nodes, uint32_t nn,
+                                                 uint32_t* __restrict__ parent, uint32_t* __restrict__ topid) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nn) return;
+    if (i == 0) parent[0] = kNone;
+    topid[i] = kNone;
+    if (is_branch(nodes[i])) {
+        parent[nodes[i].left] = i;
+        parent[nodes[i].right] = i;
+    }
+}
+__global__ void __launch_bounds__(256) k_top_ids(const uint32_t* __restrict__ top, uint32_t ntop,
+                                                 uint32_t* __restrict__ topid) {
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < ntop) topid[top[k]] = k;
+}
+
+// flag: a record's node outside the top list (a branch at an even depth, counted up the parents).
+// *odd_boxes is set when a box is not finite or not ordered.
+__global__ void __launch_bounds__(256) k_record_flags(const BuildNode* __restrict__ nodes, uint32_t nn,
+                                                      const uint32_t* __restrict__ parent,
+                                                      const uint32_t* __restrict__ topid, uint32_t* __restrict__ flag,
+                                                      uint32_t* __restrict__ odd_boxes) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i > nn) return;
+    uint32_t f = 0;
+    if (i < nn) {
+        const BuildNode n = nodes[i];
+        bool ok = true;
+        for (int k = 0; k < 3; ++k)
+            ok = ok && __builtin_isfinite(n.bmin[k]) && __builtin_isfinite(n.bmax[k]) && n.bmin[k] <= n.bmax[k];
+        if (!ok) atomicOr(odd_boxes, 1u);
+        if (is_branch(n) && topid[i] == kNone) {
+            uint32_t depth = 0;
+            for (uint32_t p = parent[i]; p != kNone; p = parent[p]) ++depth;
+            f = (depth & 1u) ^ 1u;
+        }
+    }
+    flag[i] = f;
+}
+
+// Whether a branch's right child comes first, a bit per direction class. The six direction sorts
+// are applied one after another to the same tree, as common/threaded_bvh.hpp:518-525 does, so a
+// child pair whose centres tie is swapped by every sort.
+__device__ uint32_t child_orders(const BuildNode& n, const BuildNode* __restrict__ nodes) {
+    uint32_t bits = 0;
+    if (!is_branch(n)) return bits;
+    bool swapped = false;
+    const BuildNode l = nodes[n.left], r = nodes[n.right];
+    for (int dir = 0; dir < 6; ++dir) {
+        const int axis = dir / 2;
+        const float lc = 0.5f * (l.bmin[axis] + l.bmax[axis]), rc = 0.5f * (r.bmin[axis] + r.bmax[axis]);
+        const float first = swapped != ((dir & 1) != 0) ? rc : lc, second = swapped != ((dir & 1) != 0) ? lc : rc;
+        if (!(first < second)) swapped = !swapped;
+        bits |= (swapped ? 1u : 0u) << dir;
+    }
+    return bits;
+}
+
+__global__ void __launch_bounds__(256) k_pack_records(const BuildNode* __restrict__ nodes, uint32_t nn,
+                                                      const uint32_t* __restrict__ topid,
+                                                      const uint32_t* __restrict__ flag,
+                                                      const uint32_t* __restrict__ rank, uint32_t ntop,
+                                                      WalkNode* __restrict__ out) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nn || (topid[i] == kNone && flag[i] == 0)) return;
+    auto record = [&](uint32_t x) { return topid[x] != kNone ? topid[x] : ntop + rank[x]; };
+    const BuildNode n = nodes[i];
+    WalkNode w;
+    w.order = 0;
+    uint32_t orders[3];
+    orders[0] = child_orders(n, nodes);
+    for (int h = 0; h < 2; ++h) {
+        const uint32_t c = (uint32_t)(h == 0 ? n.left : n.right);
+        const BuildNode child = nodes[c];
+        orders[1 + h] = child_orders(child, nodes);
+        const bool leaf = !is_branch(child);  // a leaf child: its own box twice, no second link
+        for (int k = 0; k < 2; ++k) {
+            const uint32_t g = leaf ? c : (uint32_t)(k == 0 ? child.left : child.right);
+            const BuildNode b = nodes[g];
+            for (int a = 0; a < 3; ++a) {
+                w.box[2 * h + k][a] = b.bmin[a];
+                w.box[2 * h + k][3 + a] = b.bmax[a];
+            }
+            w.link[2 * h + k] = leaf && k == 1 ? kInvalid : (is_branch(b) ? 8u * record(g) : leaf_word(b));
+        }
+    }
+    for (int dir = 0; dir < 6; ++dir)
+        for (int k = 0; k < 3; ++k) w.order |= ((orders[k] >> dir) & 1u) << (3 * dir + k);
+    for (int k = 0; k < 3; ++k) w.pad[k] = 0;
+    out[record(i)] = w;
+}
+
+__global__ void __launch_bounds__(256) k_pack_prims(const uint32_t* __restrict__ prim_ids, uint32_t nslots,
+                                                    const float* __restrict__ points, uint32_t stride,
+                                                    const uint32_t* __restrict__ indices, uint32_t ntris,
+                                                    const float* __restrict__ spheres, PrimRec* __restrict__ out) {
+    const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
+    if (slot >= nslots) return;
+    const uint32_t p = prim_ids[slot];
+    PrimRec r = {};
+    r.prim = p;
+    if (p < ntris) {
+        float v[3][3];
+        for (int j = 0; j < 3; ++j) {
+            const float* q = points + (size_t)indices[3 * (size_t)p + j] * stride;
+            for (int k = 0; k < 3; ++k) v[j][k] = q[k];
+        }
+        r.q0[0] = v[0][0];
+        r.q0[1] = v[0][1];
+        r.q0[2] = v[0][2];
+        r.q0[3] = v[1][0] - v[0][0];
+        r.q1[0] = v[1][1] - v[0][1];
+        r.q1[1] = v[1][2] - v[0][2];
+        r.q1[2] = v[2][0] - v[0][0];
+        r.q1[3] = v[2][1] - v[0][1];
+        r.e2z = v[2][2] - v[0][2];
+    } else {
+        for (int k = 0; k < 4; ++k) r.q0[k] = spheres[4 * (size_t)(p - ntris) + k];
+    }
+    out[slot] = r;
+}
+
+__global__ void __launch_bounds__(256) k_points4(const float* __restrict__ points, uint32_t stride, uint32_t npoints,
+                                                 float4* __restrict__ out) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= npoints) return;
+    const float* p = points + (size_t)i * stride;
+    out[i] = make_float4(p[0], p[1], p[2], 0.0f);
+}
+
+inline dim3 blocks_of(size_t n) { return dim3((uint32_t)((n + 255) / 256)); }
+
+// The first `count` record nodes in breadth-first order (the tree is not a single leaf).
+std::vector<uint32_t> top_records(const std::vector<BuildNode>& nodes, size_t count) {
+    std::vector<uint32_t> order{0};
+    for (size_t h = 0; h < order.size() && order.size() < count; ++h) {
+        for (const int32_t c : {nodes[order[h]].left, nodes[order[h]].right}) {
+            if (nodes[c].left < 0) continue;
+            for (const int32_t g : {nodes[c].left, nodes[c].right})
+                if (nodes[g].left >= 0 && order.size() < count) order.push_back((uint32_t)g);
+        }
+    }
+    return order;
+}
+
+struct Transient {  // freed once the packing kernels are done
+    void* p = nullptr;
+    ~Transient() {
+        if (p) (void)hipFree(p);
+    }
+};
+
+}  // namespace
+
+#define PACK(call)                            \
+    do {                                      \
+        const hipError_t e_ = (call);         \
+        if (e_ != hipSuccess) return e_;      \
+    } while (0)
+
+hipError_t pack_scene(const BVHTree& t, const float* points, uint32_t stride, uint32_t npoints,
+                      const uint32_t* indices, uint32_t ntris, const float* spheres, uint32_t nspheres, hipStream_t s,
+                      SceneTables* tables, TraceScene* dev) {
+    const uint32_t nn = (uint32_t)t.nodes.size(), nslots = (uint32_t)t.prim_ids.size();
+    // one transient allocation: tree, slots, raw vertices, per-node words, scan space
+    const size_t words = (size_t)nn + 1;
+    size_t need = 0;
+    auto take = [&](size_t bytes) {
+        const size_t at = need;
+        need = (need + bytes + 255) / 256 * 256;
+        return at;
+    };
+    const size_t at_nodes = take(nn * sizeof(BuildNode)), at_ids = take((size_t)nslots * 4);
+    const size_t at_raw = take((size_t)npoints * stride * 4), at_top = take(kTreeletMaxNodes * 4);
+    const size_t at_parent = take(words * 4), at_topid = take(words * 4), at_flag = take(words * 4);
+    const size_t at_rank = take(words * 4), at_scan = take(scan_temp_words(words) * 4), at_odd = take(4);
+    Transient tmp;
+    PACK(hipMalloc(&tmp.p, need));
+    char* const base = static_cast<char*>(tmp.p);
+    auto at = [&](size_t off) { return reinterpret_cast<uint32_t*>(base + off); };
+    const BuildNode* nodes = reinterpret_cast<const BuildNode*>(base + at_nodes);
+    const float* raw = reinterpret_cast<const float*>(base + at_raw);
+
+    std::vector<uint32_t> top;
+    const bool records = nn != 0 && t.nodes[0].left >= 0;
+    uint32_t nwalk = 0, odd = 0;
+    if (nn) {
+        PACK(hipMemcpyAsync(base + at_nodes, t.nodes.data(), nn * sizeof(BuildNode), hipMemcpyHostToDevice, s));
+        if (records) top = top_records(t.nodes, kTreeletMaxNodes);
+        const uint32_t ntop = (uint32_t)top.size();
+        if (ntop) PACK(hipMemcpyAsync(at(at_top), top.data(), (size_t)ntop * 4, hipMemcpyHostToDevice, s));
+        hipLaunchKernelGGL(k_parents, blocks_of(nn), dim3(256), 0, s, nodes, nn, at(at_parent), at(at_topid));
+        if (ntop)
+            hipLaunchKernelGGL(k_top_ids, blocks_of(ntop), dim3(256), 0, s, at(at_top), ntop, at(at_topid));
+        PACK(hipMemcpyAsync(at(at_odd), &odd, 4, hipMemcpyHostToDevice, s));
+        hipLaunchKernelGGL(k_record_flags, blocks_of(words), dim3(256), 0, s, nodes, nn, at(at_parent), at(at_topid),
+                           at(at_flag), at(at_odd));
+        PACK(hipGetLastError());
+        PACK(scan_exclusive(at(at_flag), at(at_rank), words, at(at_scan), s));
+        PACK(hipMemcpyAsync(&odd, at(at_odd), 4, hipMemcpyDeviceToHost, s));
+        PACK(hipMemcpyAsync(&nwalk, at(at_rank) + nn, 4, hipMemcpyDeviceToHost, s));
+        PACK(hipStreamSynchronize(s));
+        nwalk += ntop;
+        if (nwalk) {
+            PACK(hipMalloc(&tables->walk, (size_t)nwalk * sizeof(WalkNode)));
+            hipLaunchKernelGGL(k_pack_records, blocks_of(nn), dim3(256), 0, s, nodes, nn, at(at_topid), at(at_flag),
+                               at(at_rank), ntop, static_cast<WalkNode*>(tables->walk));
+            PACK(hipGetLastError());
+        }
+    }
+    if (npoints) {
+        PACK(hipMemcpyAsync(base + at_raw, points, (size_t)npoints * stride * 4, hipMemcpyHostToDevice, s));
+        PACK(hipMalloc(&tables->points, (size_t)npoints * 16));
+        hipLaunchKernelGGL(k_points4, blocks_of(npoints), dim3(256), 0, s, raw, stride, npoints,
+                           static_cast<float4*>(tables->points));
+        PACK(hipGetLastError());
+    }
+    if (ntris) {
+        PACK(hipMalloc(&tables->indices, (size_t)ntris * 12));
+        PACK(hipMemcpyAsync(tables->indices, indices, (size_t)ntris * 12, hipMemcpyHostToDevice, s));
+    }
+    if (nspheres) {
+        PACK(hipMalloc(&tables->spheres, (size_t)nspheres * 16));
+        PACK(hipMemcpyAsync(tables->spheres, spheres, (size_t)nspheres * 16, hipMemcpyHostToDevice, s));
+    }
+    if (nslots) {
+        PACK(hipMemcpyAsync(at(at_ids), t.prim_ids.data(), (size_t)nslots * 4, hipMemcpyHostToDevice, s));
+        PACK(hipMalloc(&tables->prims, (size_t)nslots * sizeof(PrimRec)));
+        hipLaunchKernelGGL(k_pack_prims, blocks_of(nslots), dim3(256), 0, s, at(at_ids), nslots, raw, stride,
+                           static_cast<const uint32_t*>(tables->indices), ntris,
+                           static_cast<const float*>(tables->spheres), static_cast<PrimRec*>(tables->prims));
+        PACK(hipGetLastError());
+    }
+    PACK(hipStreamSynchronize(s));
+
+    dev->walk_nodes = static_cast<const WalkNode*>(tables->walk);
+    dev->nwalk = nwalk;
+    dev->root = nn == 0 || records ? 0u : kLeafFlag | ((t.nodes[0].prim_cnt - 1) << 28) | t.nodes[0].prim_beg;
+    dev->prims = static_cast<const PrimRec*>(tables->prims);
+    dev->points = static_cast<const float4*>(tables->points);
+    dev->indices = static_cast<const uint32_t*>(tables->indices);
+    dev->spheres = static_cast<const float4*>(tables->spheres);
+    dev->nnodes = nn;
+    dev->sphere_begin = (int32_t)ntris;
+    dev->boxes_finite = odd == 0 ? 1u : 0u;
+    for (int k = 0; nn != 0 && k < 3; ++k) {
+        dev->root_lo[k] = t.nodes[0].bmin[k];
+        dev->root_hi[k] = t.nodes[0].bmax[k];
+    }
+    return hipSuccess;
+}
+
+}  // namespace rgpu

@@ -1,0 +1,54 @@
+"""The scene fingerprint that checkpoints compare: made piece by piece on several threads, it must
+stay the fingerprint of the whole record arrays (so that old snapshots still resume)."""
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "raccoongpurender_amd", "csrc")
+
+PROGRAM = r"""
+#include <cstdio>
+#include <random>
+#include "bvh_build.h"
+#include "fingerprint.h"
+using namespace rgpu;
+int main(int argc, char** argv) {
+    const uint32_t ntris = atoi(argv[1]), nsph = atoi(argv[2]), top = atoi(argv[3]);
+    std::mt19937 rng(7);
+    std::uniform_real_distribution<float> U(0.0f, 1.0f);
+    std::vector<float> pts, sph;
+    std::vector<uint32_t> idx;
+    for (uint32_t i = 0; i < 9 * ntris; ++i) pts.push_back(U(rng));
+    for (uint32_t i = 0; i < 3 * ntris; ++i) idx.push_back(i);
+    for (uint32_t i = 0; i < 4 * nsph; ++i) sph.push_back(0.1f * U(rng));
+    BVHTree t;
+    build_bvh(pts.data(), 3, 3 * ntris, idx.data(), ntris, sph.data(), nsph, BuildOptions(), &t);
+    std::vector<SLNode> sl;
+    pack_stackless(t, &sl);
+    number_top_breadth_first(&sl, top);
+    mark_leaf_links(&sl);
+    std::vector<PrimRec> pr(t.prim_ids.size());
+    pack_prims(t, pts.data(), 3, idx.data(), ntris, sph.data(), 0, pr.size(), pr.data());
+    const uint64_t want = fingerprint64(pr.data(), pr.size() * sizeof(PrimRec),
+                                        fingerprint64(sl.data(), sl.size() * sizeof(SLNode), ntris));
+    for (uint32_t threads : {1u, 3u, 8u})
+        if (scene_fingerprint(t, top, pts.data(), 3, idx.data(), ntris, sph.data(), threads) != want) return 1;
+    return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    d = tmp_path_factory.mktemp("fp")
+    (d / "fp.cpp").write_text(PROGRAM)
+    subprocess.check_call(["g++", "-std=c++17", "-O2", "-I" + CSRC, "-o", str(d / "fp"), str(d / "fp.cpp"),
+                           os.path.join(CSRC, "bvh_build.cpp"), "-lpthread"])
+    return str(d / "fp")
+
+
+@pytest.mark.parametrize("ntris,nspheres,top", [(0, 0, 1024), (1, 0, 1024), (2, 1, 1024), (700, 5, 1024), (3000, 0, 1024),
+                                                (60000, 33, 1024), (3000, 0, 1)])
+def test_piecewise_equals_whole(program, ntris, nspheres, top):
+    assert subprocess.run([program, str(ntris), str(nspheres), str(top)]).returncode == 0
