@@ -42,8 +42,9 @@ static const uint32_t kChildLeaf = 0x40000000u;
 static const uint32_t kInvalid = 0xFFFFFFFFu;
 
 // Record of the walk on the device, one 128-byte line per branch node at an even depth: the boxes
-// of its four grandchildren (6 floats each, min xyz then max xyz; left child's first), their links
-// and the child orders. A link is
+// of its four grandchildren (left child's first), their links and the child orders. The planes lie
+// by axis, the four lower ones in one 16-byte word and the upper ones in the next, so that a ray
+// reads the near and the far planes of an axis by its sign. A link is
 //   a branch's   8 * its record's id (the record's index in 16-byte units); kFirstHalf or
 //                kSecondHalf added means that child of the record's node alone, kOneBox + k its
 //                k-th box alone;
@@ -55,7 +56,7 @@ static const uint32_t kInvalid = 0xFFFFFFFFu;
 // BVH (common/threaded_bvh.hpp:494-525): whether the right child comes first, and the same for the
 // left and the right child's children. These 18 bits hold what six pre-ordered node tables held.
 struct alignas(128) WalkNode {
-    float box[4][6];
+    float planes[6][4];  // x lower, x upper, y lower, ...
     uint32_t link[4];
     uint32_t order;
     uint32_t pad[3];

@@ -104,8 +104,8 @@ __global__ void __launch_bounds__(256) k_pack_records(const BuildNode* __restric
             const uint32_t g = leaf ? c : (uint32_t)(k == 0 ? child.left : child.right);
             const BuildNode b = nodes[g];
             for (int a = 0; a < 3; ++a) {
-                w.box[2 * h + k][a] = b.bmin[a];
-                w.box[2 * h + k][3 + a] = b.bmax[a];
+                w.planes[2 * a][2 * h + k] = b.bmin[a];
+                w.planes[2 * a + 1][2 * h + k] = b.bmax[a];
             }
             w.link[2 * h + k] = leaf && k == 1 ? kInvalid : (is_branch(b) ? 8u * record(g) : leaf_word(b));
         }

@@ -22,17 +22,12 @@ __device__ __forceinline__ F3 cross3(F3 a, F3 b) {
 }
 
 // One axis of the slab test: entry/exit parameters with the NaN substitution of
-// kernels/slab.cl:15-16 (t0 first, then t1 from the updated t0). kPlain leaves the
-// substitution out; callers choose it only where neither product can be NaN, so both forms
-// give the same bits there.
-template <bool kPlain = false>
+// kernels/slab.cl:15-16 (t0 first, then t1 from the updated t0).
 __device__ __forceinline__ void slab_axis(float lo, float hi, float o, float inv, float* tn, float* tf) {
     float t0 = (lo - o) * inv;
     float t1 = (hi - o) * inv;
-    if (!kPlain) {
-        t0 = __builtin_isnan(t0) ? -t1 : t0;
-        t1 = __builtin_isnan(t1) ? -t0 : t1;
-    }
+    t0 = __builtin_isnan(t0) ? -t1 : t0;
+    t1 = __builtin_isnan(t1) ? -t0 : t1;
     *tn = fminf(t0, t1);
     *tf = fmaxf(t0, t1);
 }
@@ -175,7 +170,10 @@ __device__ __forceinline__ uint32_t direction_class(F3 rd) {
 // and a stack whose push and pop are one LDS access: 1.00 ms. One 128-byte line for two levels,
 // none for leaves: 0.77 ms, 13.5 visits a ray, 5,800 VALU operations (76 % busy at 48 %), 3.4 GB
 // (4.4 TB/s). Both bounds are near; 8 waves per SIMD fetch more from beyond the L2 and are
-// slower. Threaded: seven pre-ordered tables of 32-byte records (344 MB for that scene, 51.7 visits
+// slower. Near and far planes by address, in place of a minimum and a maximum per box and axis, and
+// the visit's kind as a scalar took another 5 % off these rays (0.84 -> 0.80 ms with the launch) and
+// 3 to 5 % off the wavefront's stage (4.19 M slots: 1.33 -> 1.28 ms; with the signs' offsets in
+// registers of their own, which then spill, 1.40). Threaded: seven pre-ordered tables of 32-byte records (344 MB for that scene, 51.7 visits
 // a ray, 9.3 GB from beyond the L2 a launch) took 2.04 ms by direction class and 1.97 ms in the
 // tree's own order; the records that the stackless walk reads, with the child orders as bits, take
 // 0.90 and 1.09 ms, and the tables are gone from the scene (327,680 triangles: 57 -> 20 ms).
@@ -247,7 +245,7 @@ __device__ __forceinline__ int32_t visit_kind(const WalkRay& r, bool boxes_finit
 }
 // The same after primitive tests, which only change clips.
 __device__ __forceinline__ int32_t visit_kind_after(int32_t kind, const WalkRay& r) {
-    return __all(r.tmin == r.tmin) ? kind : (int32_t)kVisitBinary;
+    return wave_scalar(__all(r.tmin == r.tmin) ? kind : (int32_t)kVisitBinary);
 }
 
 // Stages the first `top` records at the start of walk_lds (the whole workgroup; barrier after).
@@ -260,6 +258,9 @@ __device__ __forceinline__ void stage_records(const float4* __restrict__ recs, u
     }
     __syncthreads();
 }
+
+// Whether the records take more than 32 bits of byte offsets.
+__device__ __forceinline__ bool wide_records(const TraceScene& sc) { return sc.nwalk > (1u << 25); }
 
 // The two places of a record, kept apart by address space: as generic pointers the compiler
 // joins the two reads into flat loads, which go to both memories.
@@ -300,24 +301,12 @@ struct BoxSlabs {
         return Slab{fmaxf(fmaxf(n[0], n[1]), n[2]), fminf(fminf(f[0], f[1]), f[2])};
     }
 };
-// kVisitFlat: a box that a plane of an axis without motion touches spans that axis, as the
-// reference's substitution makes it; a box of no extent there, whose products are both NaN, is
-// given the same span (the reference's minima and maxima ignore the axis), so that unions of
-// intervals stay intervals of unions.
-template <int kKind>
+// The binary visit's slab test, with the reference's substitution.
 __device__ __forceinline__ BoxSlabs box_slabs(const BoxPlanes& b, F3 o, F3 inv) {
     BoxSlabs s;
-    const float oo[3] = {o.x, o.y, o.z}, ii[3] = {inv.x, inv.y, inv.z};
-    for (int k = 0; k < 3; ++k) {
-        if (kKind == kVisitFlat) {
-            const float t0 = (b.lo[k] - oo[k]) * ii[k], t1 = (b.hi[k] - oo[k]) * ii[k];
-            const bool touch = __builtin_isunordered(t0, t1);
-            s.n[k] = touch ? -__builtin_inff() : fminf(t0, t1);
-            s.f[k] = touch ? __builtin_inff() : fmaxf(t0, t1);
-        } else {
-            slab_axis<kKind == kVisitPlain>(b.lo[k], b.hi[k], oo[k], ii[k], &s.n[k], &s.f[k]);
-        }
-    }
+    slab_axis(b.lo[0], b.hi[0], o.x, inv.x, &s.n[0], &s.f[0]);
+    slab_axis(b.lo[1], b.hi[1], o.y, inv.y, &s.n[1], &s.f[1]);
+    slab_axis(b.lo[2], b.hi[2], o.z, inv.z, &s.n[2], &s.f[2]);
     return s;
 }
 __device__ __forceinline__ BoxSlabs join(const BoxSlabs& a, const BoxSlabs& b) {
@@ -337,52 +326,102 @@ __device__ __forceinline__ BoxPlanes join(const BoxPlanes& a, const BoxPlanes& b
     return s;
 }
 
+// A record as a ray sees it: per axis the four boxes' planes that it meets first (near) and last.
 struct WalkRecord {
-    BoxPlanes box[4];
+    WalkWords near[3], far[3];
     WalkLinks link;
     uint32_t order;  // kVariantThreaded
 };
-// kTop: records below link `top8` (8 * records) come from LDS.
+// kTop: records below link `top8` (8 * records) come from LDS. Which of an axis's two plane words
+// is the near one, the ray's sign tells the address: no minimum or maximum per box and axis (inv 0:
+// the lower planes are near). sign: 27, the shift from a float's sign to a plane word's bytes. Byte offsets of 32 bits into the records (a scalar base and one
+// register for each address); wide: a scene of more than 4 GiB of them.
 template <bool kTop, int kVariant>
-__device__ __forceinline__ void load_record(uint32_t at, const float4* __restrict__ recs, uint32_t top8, WalkRecord* r) {
-    WalkWords q[6];
+__device__ __forceinline__ void load_record(uint32_t at, const float4* __restrict__ recs, uint32_t top8, bool wide,
+                                            F3 inv, uint32_t sign, WalkRecord* r) {
+    // 16 (a plane word's bytes) where the ray runs against the axis, else 0
+    const uint32_t n0 = __float_as_uint(inv.x) >> sign & 16u, n1 = __float_as_uint(inv.y) >> sign & 16u,
+                   n2 = __float_as_uint(inv.z) >> sign & 16u;
     if (kTop && at < top8) {
-        const auto* p = (const LdsSpace WalkWords*)((const LdsSpace char*)walk_lds + __umul24(at, kStagedBytes / 8u));
-        for (int k = 0; k < 6; ++k) q[k] = p[k];
-        r->link = *(const LdsSpace WalkLinks*)(p + 6);
+        const uint32_t a = __umul24(at, kStagedBytes / 8u) + (uint32_t)(uintptr_t)(const LdsSpace char*)walk_lds;
+        auto word = [](uint32_t x) { return (const LdsSpace char*)(uintptr_t)x; };
+        r->near[0] = *(const LdsSpace WalkWords*)(word(a + n0));
+        r->far[0] = *(const LdsSpace WalkWords*)(word(a - n0) + 16);
+        r->near[1] = *(const LdsSpace WalkWords*)(word(a + n1) + 32);
+        r->far[1] = *(const LdsSpace WalkWords*)(word(a - n1) + 48);
+        r->near[2] = *(const LdsSpace WalkWords*)(word(a + n2) + 64);
+        r->far[2] = *(const LdsSpace WalkWords*)(word(a - n2) + 80);
+        r->link = *(const LdsSpace WalkLinks*)(word(a) + 96);
         if constexpr (kVariant == kVariantThreaded)
             r->order = *(const LdsSpace uint32_t*)((const LdsSpace char*)walk_lds + __umul24(top8, kStagedBytes / 8u) + at / 2u);
+    } else if (!wide) {
+        const uint32_t a = at << 4;
+        const auto* p = (const GlobalSpace char*)recs;
+        r->near[0] = *(const GlobalSpace WalkWords*)(p + (a | n0));
+        r->far[0] = *(const GlobalSpace WalkWords*)(p + ((a | n0) ^ 16u));
+        r->near[1] = *(const GlobalSpace WalkWords*)(p + (a | n1) + 32);
+        r->far[1] = *(const GlobalSpace WalkWords*)(p + ((a | n1) ^ 16u) + 32);
+        r->near[2] = *(const GlobalSpace WalkWords*)(p + (a | n2) + 64);
+        r->far[2] = *(const GlobalSpace WalkWords*)(p + ((a | n2) ^ 16u) + 64);
+        r->link = *(const GlobalSpace WalkLinks*)(p + a + 96);
+        if constexpr (kVariant == kVariantThreaded) r->order = *(const GlobalSpace uint32_t*)(p + a + 112);
     } else {
-        const auto* p = (const GlobalSpace WalkWords*)recs + at;
-        for (int k = 0; k < 6; ++k) q[k] = p[k];
-        r->link = *(const GlobalSpace WalkLinks*)(p + 6);
-        if constexpr (kVariant == kVariantThreaded) r->order = *(const GlobalSpace uint32_t*)(p + 7);
+        // (records are 128-byte aligned: a plane's offset goes into the address' low word)
+        const uint64_t a = (uint64_t)(uintptr_t)recs + ((uint64_t)at << 4);
+        const uint32_t lo = (uint32_t)a, hi = (uint32_t)(a >> 32);
+        auto word = [hi](uint32_t x) { return (const GlobalSpace char*)(uintptr_t)((uint64_t)hi << 32 | x); };
+        r->near[0] = *(const GlobalSpace WalkWords*)(word(lo | n0));
+        r->far[0] = *(const GlobalSpace WalkWords*)(word((lo | n0) ^ 16u));
+        r->near[1] = *(const GlobalSpace WalkWords*)(word(lo | n1) + 32);
+        r->far[1] = *(const GlobalSpace WalkWords*)(word((lo | n1) ^ 16u) + 32);
+        r->near[2] = *(const GlobalSpace WalkWords*)(word(lo | n2) + 64);
+        r->far[2] = *(const GlobalSpace WalkWords*)(word((lo | n2) ^ 16u) + 64);
+        r->link = *(const GlobalSpace WalkLinks*)(word(lo) + 96);
+        if constexpr (kVariant == kVariantThreaded) r->order = *(const GlobalSpace uint32_t*)(word(lo) + 112);
     }
-    for (int h = 0; h < 2; ++h) {
-        const WalkWords a = q[3 * h], b = q[3 * h + 1], c = q[3 * h + 2];
-        r->box[2 * h] = BoxPlanes{{a.x, a.y, a.z}, {a.w, b.x, b.y}};
-        r->box[2 * h + 1] = BoxPlanes{{b.z, b.w, c.x}, {c.y, c.z, c.w}};
+}
+// Box k of a record loaded with near planes (of ordered boxes: the products of the near planes are
+// the smaller ones, rounding included).
+// kVisitFlat: a box that a plane of an axis without motion touches spans that axis, as the
+// reference's substitution makes it; a box of no extent there, whose products are both NaN, is
+// given the same span (the reference's minima and maxima ignore the axis), so that unions of
+// intervals stay intervals of unions.
+template <int kKind>
+__device__ __forceinline__ BoxSlabs record_slabs(const WalkRecord& w, int k, F3 o, F3 inv) {
+    BoxSlabs s;
+    const float oo[3] = {o.x, o.y, o.z}, ii[3] = {inv.x, inv.y, inv.z};
+    for (int a = 0; a < 3; ++a) {
+        s.n[a] = (w.near[a][k] - oo[a]) * ii[a];
+        s.f[a] = (w.far[a][k] - oo[a]) * ii[a];
+        if (kKind == kVisitFlat) {
+            const bool touch = __builtin_isunordered(s.n[a], s.f[a]);
+            s.n[a] = touch ? -__builtin_inff() : s.n[a];
+            s.f[a] = touch ? __builtin_inff() : s.f[a];
+        }
     }
+    return s;
 }
 
 // Visit of the record `node` names: descent two levels down, what else is hit deferred, or a pop
 // when nothing is hit. kKind: kVisitPlain or kVisitFlat.
 template <int kVariant, bool kTop, int kKind>
 __device__ __forceinline__ void walk_visit(WalkRay& r, const WalkStack& stk, const float4* __restrict__ recs,
-                                           uint32_t top8) {
+                                           uint32_t top8, bool wide) {
     constexpr bool kNear = kVariant == kVariantStackless;  // else in the order of the tables
     uint32_t at = r.node & ~7u;
     const uint32_t only = r.node & 7u;  // kFirstHalf, kSecondHalf, kOneBox + k or 0
     // (an opaque, different start keeps the compiler from joining the two kinds' common part,
-    // which would hold all 24 products of a record in registers)
-    if (kKind == kVisitPlain) asm("; plain visit" : "+v"(at));
-    else asm("; flat visit" : "+v"(at));
+    // which would hold all 24 products of a record in registers, and an opaque shift the signs' offsets
+    // from taking registers over the whole walk)
+    uint32_t sign = 27;
+    if (kKind == kVisitPlain) asm("; plain visit" : "+v"(at), "+s"(sign));
+    else asm("; flat visit" : "+v"(at), "+s"(sign));
     WalkRecord w;
-    load_record<kTop, kVariant>(at, recs, top8, &w);
-    const BoxSlabs s0 = box_slabs<kKind>(w.box[0], r.ro, r.inv), s1 = box_slabs<kKind>(w.box[1], r.ro, r.inv);
+    load_record<kTop, kVariant>(at, recs, top8, wide, r.inv, sign, &w);
+    const BoxSlabs s0 = record_slabs<kKind>(w, 0, r.ro, r.inv), s1 = record_slabs<kKind>(w, 1, r.ro, r.inv);
     Span c0 = clipped(s0.clip(), r.tmin), c1 = clipped(s1.clip(), r.tmin);
     const Span L = clipped(join(s0, s1).clip(), r.tmin);
-    const BoxSlabs s2 = box_slabs<kKind>(w.box[2], r.ro, r.inv), s3 = box_slabs<kKind>(w.box[3], r.ro, r.inv);
+    const BoxSlabs s2 = record_slabs<kKind>(w, 2, r.ro, r.inv), s3 = record_slabs<kKind>(w, 3, r.ro, r.inv);
     Span c2 = clipped(s2.clip(), r.tmin), c3 = clipped(s3.clip(), r.tmin);
     const Span R = clipped(join(s2, s3).clip(), r.tmin);
     // what the link leaves out is not hit
@@ -442,12 +481,14 @@ __device__ __forceinline__ float pick(float a, float b, float c, float d, uint32
     const float l = (k & 1u) ? b : a, h = (k & 1u) ? d : c;
     return (k & 2u) ? h : l;
 }
+// Box k of a record loaded with the lower planes near.
 __device__ __forceinline__ BoxPlanes pick_box(const WalkRecord& w, uint32_t k) {
-    const BoxPlanes a = w.box[0], b = w.box[1], c = w.box[2], d = w.box[3];
-    return BoxPlanes{{pick(a.lo[0], b.lo[0], c.lo[0], d.lo[0], k), pick(a.lo[1], b.lo[1], c.lo[1], d.lo[1], k),
-                      pick(a.lo[2], b.lo[2], c.lo[2], d.lo[2], k)},
-                     {pick(a.hi[0], b.hi[0], c.hi[0], d.hi[0], k), pick(a.hi[1], b.hi[1], c.hi[1], d.hi[1], k),
-                      pick(a.hi[2], b.hi[2], c.hi[2], d.hi[2], k)}};
+    BoxPlanes b;
+    for (int a = 0; a < 3; ++a) {
+        b.lo[a] = pick(w.near[a].x, w.near[a].y, w.near[a].z, w.near[a].w, k);
+        b.hi[a] = pick(w.far[a].x, w.far[a].y, w.far[a].z, w.far[a].w, k);
+    }
+    return b;
 }
 __device__ __forceinline__ uint32_t pick_link(const WalkRecord& w, uint32_t k) {
     const uint32_t l = (k & 1u) ? w.link.y : w.link.x, h = (k & 1u) ? w.link.w : w.link.z;
@@ -460,15 +501,16 @@ __device__ __forceinline__ uint32_t pick_link(const WalkRecord& w, uint32_t k) {
 // boxes), then each entered half.
 template <bool kTop, bool kCount>
 __device__ __forceinline__ void stackless_visit_binary(WalkRay& r, const WalkStack& stk,
-                                                       const float4* __restrict__ recs, uint32_t top8, Cnt* cnt) {
+                                                       const float4* __restrict__ recs, uint32_t top8, bool wide,
+                                                       Cnt* cnt) {
     const uint32_t at = r.node & ~7u, only = r.node & 7u;
     WalkRecord w;
-    load_record<kTop, kVariantStackless>(at, recs, top8, &w);
+    load_record<kTop, kVariantStackless>(at, recs, top8, wide, f3(0.0f, 0.0f, 0.0f), 27u, &w);
     BoxPlanes A, B;
     uint32_t la, lb;
     if (only == 0) {
-        A = join(w.box[0], w.box[1]);
-        B = join(w.box[2], w.box[3]);
+        A = join(pick_box(w, 0), pick_box(w, 1));
+        B = join(pick_box(w, 2), pick_box(w, 3));
         // a leaf child of the node is entered by its word
         la = w.link.y == kInvalid ? w.link.x : at | kFirstHalf;
         lb = w.link.w == kInvalid ? w.link.z : at | kSecondHalf;
@@ -479,7 +521,7 @@ __device__ __forceinline__ void stackless_visit_binary(WalkRay& r, const WalkSta
         la = pick_link(w, k);
         lb = pick_link(w, k + 1u);
     }
-    const Slab a = box_slabs<kVisitBinary>(A, r.ro, r.inv).clip(), b = box_slabs<kVisitBinary>(B, r.ro, r.inv).clip();
+    const Slab a = box_slabs(A, r.ro, r.inv).clip(), b = box_slabs(B, r.ro, r.inv).clip();
     const bool ha = a.hit(r.tmin), hb = b.hit(r.tmin);
     const bool takeA = ha && (!hb || nearer(clipped(a, r.tmin), clipped(b, r.tmin)));
     if (kCount) {
@@ -495,14 +537,15 @@ __device__ __forceinline__ void stackless_visit_binary(WalkRay& r, const WalkSta
 // a second grandchild as its box.
 template <int kVariant, bool kTop, bool kCount>
 __device__ __forceinline__ void threaded_visit_binary(WalkRay& r, const WalkStack& stk,
-                                                      const float4* __restrict__ recs, uint32_t top8, Cnt* cnt) {
+                                                      const float4* __restrict__ recs, uint32_t top8, bool wide,
+                                                       Cnt* cnt) {
     const uint32_t at = r.node & ~7u, only = r.node & 7u;
     WalkRecord w;
-    load_record<kTop, kVariant>(at, recs, top8, &w);
+    load_record<kTop, kVariant>(at, recs, top8, wide, f3(0.0f, 0.0f, 0.0f), 27u, &w);
     const uint32_t turns = kVariant == kVariantThreaded ? w.order >> r.turn : 0u;
     auto test = [&](const BoxPlanes& b) {
         if (kCount) cnt->node++;
-        return box_slabs<kVisitBinary>(b, r.ro, r.inv).clip().hit(r.tmin);
+        return box_slabs(b, r.ro, r.inv).clip().hit(r.tmin);
     };
     uint32_t k = only & 3u;  // the box to test last
     bool passed;             // whether the half that holds it is entered
@@ -535,13 +578,14 @@ __device__ __forceinline__ void threaded_visit_binary(WalkRay& r, const WalkStac
 
 template <int kVariant, bool kTop, bool kCount>
 __device__ __forceinline__ void walk_visit_as(int32_t kind, WalkRay& r, const WalkStack& stk,
-                                              const float4* __restrict__ recs, uint32_t top, Cnt* cnt) {
-    if (!kCount && kind == kVisitPlain) walk_visit<kVariant, kTop, kVisitPlain>(r, stk, recs, 8 * top);
-    else if (!kCount && kind == kVisitFlat) walk_visit<kVariant, kTop, kVisitFlat>(r, stk, recs, 8 * top);
+                                              const float4* __restrict__ recs, uint32_t top, bool wide, Cnt* cnt) {
+    kind = wave_scalar(kind);  // it sits in a vector register over the walk
+    if (!kCount && kind == kVisitPlain) walk_visit<kVariant, kTop, kVisitPlain>(r, stk, recs, 8 * top, wide);
+    else if (!kCount && kind == kVisitFlat) walk_visit<kVariant, kTop, kVisitFlat>(r, stk, recs, 8 * top, wide);
     else if constexpr (kVariant == kVariantStackless)
-        stackless_visit_binary<kTop, kCount>(r, stk, recs, 8 * top, cnt);
+        stackless_visit_binary<kTop, kCount>(r, stk, recs, 8 * top, wide, cnt);
     else
-        threaded_visit_binary<kVariant, kTop, kCount>(r, stk, recs, 8 * top, cnt);
+        threaded_visit_binary<kVariant, kTop, kCount>(r, stk, recs, 8 * top, wide, cnt);
 }
 
 template <int kVariant, bool kCount>
@@ -561,7 +605,7 @@ __device__ __forceinline__ void walk_begin(WalkRay& r, const WalkStack& stk, con
     if constexpr (kVariant != kVariantStackless) {
         r.turn = 3u * direction_class(rd);
         const BoxPlanes root{{sc.root_lo[0], sc.root_lo[1], sc.root_lo[2]}, {sc.root_hi[0], sc.root_hi[1], sc.root_hi[2]}};
-        if (!box_slabs<kVisitBinary>(root, ro, r.inv).clip().hit(tmax)) r.node = kInvalid;
+        if (!box_slabs(root, ro, r.inv).clip().hit(tmax)) r.node = kInvalid;
         if (kCount) cnt->node++;
     }
 }
@@ -611,7 +655,7 @@ __device__ __forceinline__ int32_t trace_batched(const TraceScene& sc, F3 ro, F3
             if (walk_pending(st)) walk_leaf<kVariant, kCount>(st, stk, sc.prims, sc.sphere_begin, cnt);
             kind = visit_kind_after(kind, st);
         } else if (walk_walking(st)) {
-            walk_visit_as<kVariant, kTop, kCount>(kind, st, stk, recs, top, cnt);
+            walk_visit_as<kVariant, kTop, kCount>(kind, st, stk, recs, top, wide_records(sc), cnt);
         }
     }
     *tmin_io = st.tmin;

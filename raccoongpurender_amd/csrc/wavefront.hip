@@ -976,19 +976,16 @@ __device__ __forceinline__ void store_extension(const DevState& s, const TraceSc
 template <int kVariant, class J>
 __global__ void __launch_bounds__(256, 8) k_trace_step(DevState s, WFParams p, J jobs, uint32_t top) {
     const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
-    {
-        // the top `top` records of the block's scene in LDS (a job owns whole 256-slot blocks,
-        // so every slot of a workgroup traces the same scene)
-        const uint32_t first = blockIdx.x * blockDim.x;
-        const TraceScene sb = jobs.scene(jobs.job(first < p.n ? first : p.n - 1));
-        top = top < sb.nwalk ? top : sb.nwalk;
-        stage_records<kVariant>(reinterpret_cast<const float4*>(sb.walk_nodes), top);
-    }
+    // the top `top` records of the block's scene in LDS (a job owns whole 256-slot blocks, so every
+    // slot of a workgroup traces the same scene)
+    const uint32_t first = blockIdx.x * blockDim.x;
+    const uint32_t jb = jobs.job(first < p.n ? first : p.n - 1);
+    const TraceScene sc = jobs.scene(jb);
+    top = top < sc.nwalk ? top : sc.nwalk;
+    stage_records<kVariant>(reinterpret_cast<const float4*>(sc.walk_nodes), top);
     advance_cursors(s, jobs, slot);
     if (slot >= p.n) return;
     if (J::kBatch && ray_pixel(s.ray, slot) == kDeadPixel) return;
-    const uint32_t jb = jobs.job(slot);
-    const TraceScene sc = jobs.scene(jb);
     int32_t hit_volume;
     float tmin;
     volume_through(s, jobs.mats(jb), slot, &hit_volume, &tmin);
