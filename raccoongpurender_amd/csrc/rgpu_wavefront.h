@@ -195,6 +195,9 @@ struct RGB16 {
     uint32_t count;
 };
 static_assert(sizeof(RGB16) == 12, "intermediate pixel is 12 bytes");
+// rgb (3 floats a pixel) and counts of pixels [first, first + count) of 4-word accumulation records.
+hipError_t wf_split_accum(const float* accum, uint32_t first, uint32_t count, float* rgb, uint32_t* counts,
+                          hipStream_t s);
 hipError_t wf_intermediate(const DevState& st, uint32_t npixels, bool accum64, RGB16* out, hipStream_t s);
 hipError_t merge_intermediate(RGB16* a, const RGB16* b, uint32_t npixels, hipStream_t s);
 // Preview handoff (kernels/mutex.cl): words[0] the weak mutex, words[1] the step side's flag,

@@ -1290,6 +1290,25 @@ __global__ void __launch_bounds__(256) k_tonemap(DevState s, uint32_t npixels, u
     out[i] = make_uchar4(c[0], c[1], c[2], 255);
 }
 
+// Per-pixel radiance sums (3 floats a pixel) and counts out of the 4-word accumulation records, for
+// reading them back: the destination is host memory, so a workgroup's sums pass through LDS and
+// leave as whole consecutive words.
+__global__ void __launch_bounds__(256) k_split_accum(const float4* __restrict__ accum, uint32_t n,
+                                                     float* __restrict__ rgb, uint32_t* __restrict__ counts) {
+    __shared__ float sums[3 * 256];
+    const uint32_t first = blockIdx.x * 256u, t = threadIdx.x, i = first + t;
+    if (i < n) {
+        const float4 a = accum[i];
+        sums[3 * t] = a.x;
+        sums[3 * t + 1] = a.y;
+        sums[3 * t + 2] = a.z;
+        counts[i] = __float_as_uint(a.w);
+    }
+    __syncthreads();
+    const uint32_t words = 3u * min(256u, n - first);
+    for (uint32_t w = t; w < words; w += 256u) rgb[3 * (size_t)first + w] = sums[w];
+}
+
 // accumlation_to_intermediate (kernels/accumlation.cl:6-25) without its mutex: per pixel the
 // half-float mean and the sample count, widened to 32 bits.
 // held (optional): the kernel does nothing unless *held is set (copy_if_locked, kernels/mutex.cl).
@@ -1398,6 +1417,14 @@ hipError_t envmap_pdf(const DevEnvmap& e, const float* dirs, const float* normal
 hipError_t wf_tonemap(const DevState& st, uint32_t npixels, bool accum64, void* rgba8, hipStream_t s) {
     dim3 grid((npixels + 255) / 256);
     hipLaunchKernelGGL(k_tonemap, grid, dim3(256), 0, s, st, npixels, accum64 ? 1u : 0u, (uchar4*)rgba8);
+    return hipGetLastError();
+}
+
+hipError_t wf_split_accum(const float* accum, uint32_t first, uint32_t count, float* rgb, uint32_t* counts,
+                          hipStream_t s) {
+    if (count == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_split_accum, dim3((count + 255) / 256), dim3(256), 0, s,
+                       reinterpret_cast<const float4*>(accum) + first, count, rgb, counts);
     return hipGetLastError();
 }
 

@@ -1,0 +1,39 @@
+"""A batch job's image (rgpu_wavefront_job_accumulation) against a single render's.
+
+The readback passes through pinned memory 2^18 pixels at a time, 256 a workgroup: images of one
+pixel, of a workgroup and its neighbours, of one chunk exactly and of one more row, in one batch so
+that the chunk is the largest job's. Counts equal a single render's with the same seed; sums agree to
+the order of the float additions of a few samples a pixel (each at most 2^-23 relative).
+"""
+import numpy as np
+import pytest
+
+from raccoongpurender_amd import _lib, render_scenes as R
+from tests import wf_helpers as W
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("sizes", [[(1, 1), (17, 15), (16, 16), (257, 1)], [(512, 512), (3, 5)], [(512, 513), (1, 1)]])
+def test_readback_sizes(ctx, sizes):
+    jobs, keep = [], []
+    for k, (w, h) in enumerate(sizes):
+        sd = R.cornell_box(w, h, segments=8, rings=4)
+        bvh = _lib.BVH(sd["points"], sd["indices"])
+        d = (_lib.Scene(ctx, bvh), _lib.Materials(ctx, sd["materials"]), _lib.Envmap(ctx, sd["env"]))
+        keep.append((bvh, d))
+        jobs.append(_lib.BatchJob(*d, W.camera(sd["camera"]), max(256, w * h), seed=5 + k))
+    batch = _lib.Batch(ctx, jobs)
+    batch.step(6)
+    for k, j in enumerate(jobs):
+        print(f"case readback {sizes[k]}", flush=True)
+        single = _lib.Wavefront(ctx, j.scene, j.materials, j.envmap, j.slots, seed=j.seed)
+        single.initialize(j.camera)
+        single.step(6)
+        rgb, cnt = batch.job_accumulation(k)
+        rs, ns = single.accumulation()
+        assert cnt.sum() > 0 and np.array_equal(cnt, ns)
+        assert np.all(np.abs(rgb - rs) <= 1e-5 * np.abs(rs) + 1e-6)
+        again, _ = batch.job_accumulation(k)
+        assert np.array_equal(again.view(np.uint32), rgb.view(np.uint32))
+        single.close()
