@@ -117,6 +117,9 @@ struct DevEnvmap {
     uint32_t width = 0, height = 0;
 };
 
+// Words from one queue's block totals to the next's (16-byte aligned rows).
+__host__ __device__ inline uint32_t totals_stride(uint32_t nblocks) { return (nblocks + 3u) & ~3u; }
+
 struct DevState {
     TraceRay* ray = nullptr;  // ro, tmax, rd, pixel index
     PathRec* path = nullptr;
@@ -127,7 +130,8 @@ struct DevState {
     uint8_t* qsel = nullptr;          // queue chosen by logic
     uint32_t* items = nullptr;        // kNumQueues * n queue items
     uint32_t* counts = nullptr;       // kNumQueues counts
-    uint32_t* block_counts = nullptr; // kNumQueues * nblocks
+    uint32_t* block_totals = nullptr; // a bounce's items per queue and 256-slot block, rows of totals_stride()
+    uint32_t* block_counts = nullptr; // kNumQueues * nblocks: their exclusive sums
     unsigned long long* next_pixel = nullptr;
     float* accum = nullptr;           // 4 floats per pixel (r, g, b, count bits) or
     double* accum64 = nullptr;        // 3 doubles per pixel + counts in accum_count

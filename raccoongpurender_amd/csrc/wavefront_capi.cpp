@@ -207,6 +207,7 @@ int alloc_slots(rgpu_wavefront* w, size_t n) {
     s.qsel = (uint8_t*)A(n);
     s.items = (uint32_t*)A(n * kNumQueues * sizeof(uint32_t));
     s.counts = (uint32_t*)A(kNumQueues * sizeof(uint32_t));
+    s.block_totals = (uint32_t*)A((size_t)totals_stride(s.nblocks) * (kNumQueues + 1) * sizeof(uint32_t));
     s.block_counts = (uint32_t*)A((size_t)s.nblocks * (kNumQueues + 1) * sizeof(uint32_t));
     s.next_pixel = (unsigned long long*)A(sizeof(unsigned long long));
     w->stat_total = (unsigned long long*)A(sizeof(unsigned long long));
