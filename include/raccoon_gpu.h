@@ -167,7 +167,8 @@ int rgpu_extension_ray_cast(rgpu_ctx* ctx, rgpu_stream stream, const rgpu_scene*
 /* Launch shape of the persistent ray-cast kernel used when block == 0: resident waves per
  * SIMD (grid = CUs * waves_per_simd workgroups of 256; 1..16), the number of idle lanes of a
  * wave that makes it hand out its next rays (1..64), and the number of lanes waiting at leaves
- * that makes it test their primitives (1..64). 0 keeps the default (7 waves; refill at 24 idle
+ * that makes it test their primitives (1..64). 0 keeps the default (7 waves, fewer, but not below
+ * 4, where a wave would get under 64 rays; refill at 24 idle
  * lanes; leaves at 12 waiting lanes, or once as many lanes wait as walk on). leaf_batch also
  * applies to the one-thread-per-ray kernels (block != 0), whose default is 64 (leaves only once as
  * many lanes wait as walk on). treelet: the number of top-of-tree walk records each workgroup of

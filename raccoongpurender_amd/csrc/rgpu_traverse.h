@@ -57,6 +57,15 @@ struct TraceTuning {
 // lanes (8, 16: 1 % slower), 128 staged records (none: 1.04; 14 KB beside 8 KB of stacks let 7
 // workgroups share a CU's 160 KB).
 constexpr uint32_t kDefaultWaves = 7;
+// Waves per SIMD of a launch of n rays: as many as get about 64 rays each (a wave with less never
+// fills its lanes), but 4 at least. Stackless, 327,680 triangles, 4 waves against 7: 131,072 rays 144
+// and 160 us, 32,768 rays 120 and 127, 8,192 rays 95 and 95; 5 against 7: 300,000 rays 216 and 211,
+// of 5,120 triangles 89 and 103; 6 against 7: 400,000 rays 214 and 217 (102 and 100).
+constexpr uint32_t kFewestWaves = 4;
+constexpr uint32_t default_waves(uint32_t n, uint32_t cus) {
+    const uint64_t per = 64ull * 4u * cus, w = ((uint64_t)n + per / 2) / per;
+    return w < kFewestWaves ? kFewestWaves : w > kDefaultWaves ? kDefaultWaves : (uint32_t)w;
+}
 constexpr uint32_t kDefaultRefill = 24;
 constexpr uint32_t kDefaultLeafBatch = 12;
 // One thread per ray (coherent rays, the wavefront's per-slot trace): leaves wait until as many

@@ -154,7 +154,7 @@ hipError_t launch_variant(const TraceScene& sc, const TraceRay* rays, TraceHit* 
         // persistent kernel: as many resident waves as the launch asks for, each with a chunk of
         // the rays
         const uint32_t cus = tune.cu_count ? tune.cu_count : 256u;
-        const uint32_t wps = tune.waves_per_simd ? tune.waves_per_simd : kDefaultWaves;
+        const uint32_t wps = tune.waves_per_simd ? tune.waves_per_simd : default_waves(n, cus);
         const uint32_t refill = tune.refill ? tune.refill : kDefaultRefill;
         const uint32_t leaf_batch = tune.leaf_batch ? tune.leaf_batch : kDefaultLeafBatch;
         const uint32_t blocks = cus * wps;  // 4 waves (one per SIMD) per 256-thread block
