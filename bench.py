@@ -21,15 +21,17 @@ sys.path.insert(0, ROOT)
 METRIC = "Mrays/s incoherent ext. rays; equal-time relMSE guided vs plain"
 HBM_PEAK_GBS = 8000.0
 
-# Algorithmic bytes per traversal event (the record sizes the kernels fetch).
+# Algorithmic bytes per traversal event: 32 for a box test, a quarter of a 128-byte walk record (a
+# branch visit tests two boxes; a leaf's word lies in its parent's record and nothing climbs), 48 for
+# a primitive. LDS and the caches serve the upper levels, so these bytes can pass the HBM peak; the
+# roofline's rate is of the bytes moved from beyond the L2.
 RAY_IO = 32 + 16  # ray in, hit out
-SL_BRANCH, SL_LEAF, SL_PARENT, PRIM, MT_NODE = 64, 16, 16, 48, 32
+SL_BRANCH, PRIM, MT_NODE = 64, 48, 32
 
 
 def algorithmic_bytes(variant, n, c):
     if variant == "stackless":
-        return (n * RAY_IO + c["branch_visits"] * SL_BRANCH + c["leaf_visits"] * SL_LEAF
-                + c["parent_steps"] * SL_PARENT + c["prim_tests"] * PRIM)
+        return n * RAY_IO + c["branch_visits"] * SL_BRANCH + c["prim_tests"] * PRIM
     return n * RAY_IO + c["node_visits"] * MT_NODE + c["prim_tests"] * PRIM
 
 
@@ -451,8 +453,8 @@ def main():
     best = max(variants, key=lambda v: results[(v, "incoherent")]["mrays"])
     r = results[(best, "incoherent")]
     kernel = f"k_trace_persistent_{best}"
-    achieved = r["bytes"] / (r["ms"] * 1e-3) / 1e9
     traffic = read_traffic(f"{kernel}_c2_incoherent")
+    achieved = (traffic or r["bytes"]) / (r["ms"] * 1e-3) / 1e9
     out = {
         "metric": METRIC,
         "value": round(r["mrays"], 2),
@@ -484,6 +486,7 @@ def main():
             "traffic": traffic,
             "kernel": kernel,
             "algorithmic_bytes_per_launch": int(r["bytes"]),
+            "algorithmic_gbs": round(r["bytes"] / (r["ms"] * 1e-3) / 1e9, 1),
         },
         "extra": {
             f"{v}_{s}_mrays": round(results[(v, s)]["mrays"], 2) for (v, s) in results

@@ -70,7 +70,7 @@ def traversal_bytes_per_ray(ctx, scene, st, variant, sample=1 << 20):
     rd.free()
     hd.free()
     if variant == "stackless":
-        b = 64 * c["branch_visits"] + 16 * c["leaf_visits"] + 16 * c["parent_steps"]
+        b = 64 * c["branch_visits"]  # two boxes of a 128-byte walk record
     else:
         b = 32 * c["node_visits"]
     return (b + 48 * c["prim_tests"]) / n, {k: v / n for k, v in c.items()}
